@@ -153,6 +153,20 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
 }
 
+// The K loop's barrier: this wave's LDS reads have returned (another wave's
+// loads may overwrite what they read right after it), LDS accesses stay on
+// their side of it, and the loads of later stages stay in flight.  (A
+// __syncthreads is also a release fence, for which the compiler waits until
+// every LDS-DMA load of the wave has landed: the loads of stage t + 2, issued
+// at the start of stage t, then had to arrive before stage t could end.
+// Mixtral layer on MI355X with the one and the other: 2048 tokens 1805 ->
+// 1692 us, 100 tokens 561 -> 482 us.)
+__device__ __forceinline__ void stage_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // ---------------------------------------------------------------------------
 // Work decomposition.  A tile is up to 256 tokens (NRB row blocks of 32) x 256
 // weight rows; a workgroup of four waves computes it, each wave 64 rows: one
@@ -392,7 +406,7 @@ __device__ __forceinline__ void k_loop(const TileLoads& tl, int tb, int te, uint
   issue_stage<NRB>(tl, tb, lds0, wave, true);
   issue_stage<NRB>(tl, tb + 1 < te ? tb + 1 : tb, lds0 + L::kSize, wave, tb + 1 < te);
   wait_vmcnt<LPS>();
-  __syncthreads();
+  stage_barrier();
   read_b(o, tl, lds0, tb, wave, lane);
   deq_step(o, 0, 0, dr);
   read_a<NRB>(o, 0, lds0, 0, row32, h);
@@ -426,7 +440,7 @@ __device__ __forceinline__ void k_loop(const TileLoads& tl, int tb, int te, uint
       __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);  // VALU
     }
     __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
+    stage_barrier();
     __builtin_amdgcn_sched_barrier(0);
     read_a<NRB>(o, 0, nxt, 0, row32, h);  // past the last stage: unused
     __builtin_amdgcn_sched_barrier(0);
