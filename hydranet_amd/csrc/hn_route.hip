@@ -633,6 +633,17 @@ extern "C" int hn_moe_route(const void* h, long ld_h, const void* w, long ld_w, 
   const int lgv = (logits_in || w_dtype != 0 || E > 16 || H % 512 != 0 || T * E > 512)
                       ? 0 : (T <= 16 ? 1 : (T <= 32 ? 2 : (T <= 64 ? 4 : 0)));
   const bool mix = E <= 8 && k == 2 && mode == 0;
+  // Logits the MFMA path does not cover are wave dot products, which every
+  // workgroup of the routing launch would repeat for all T tokens (100 tokens
+  // x 8 experts: 119 us).  Past a few per wave they get a launch of their own,
+  // one wave each over the whole chip, and the routing reads them (same dot
+  // product, same bits; 6 + 9 us).
+  if (!logits_in && lgv == 0 && logits_out && al16(logits_out) && T * E > 256) {
+    const int rc = hn_router_logits(h, ld_h, w, ld_w, w_dtype, logits_out, T, E, H, stream);
+    if (rc) return rc;
+    logits_in = logits_out;
+    logits_out = nullptr;
+  }
 #define HN_ROUTE_LAUNCH(TW, R16, LGV, TKV)                                                          \
   hipLaunchKernelGGL((moe_route_kernel<TW, R16, LGV, TKV>), dim3(grid), dim3(kRouteThreads), 0, s, \
                      (const h16*)h, ld_h, (const TW*)w, ld_w, (const float*)logits_in,           \
