@@ -529,6 +529,7 @@ void launch_grouped(SkinnyArgs& A, const Plan& p, int E_max, hipStream_t s) {
 }
 
 constexpr int kMaxRows = 64;  // tokens per weight matrix handled per launch
+constexpr long kStreamMaxRows = 16;  // rows per matrix the streaming kernels take in one pass
 
 // Workspace layout, the same for every call: [counters: a fixed 2 MiB region
 // at the start][partials].  One buffer serves calls of every kind and size
@@ -546,6 +547,10 @@ size_t part_bytes(int ks, int mats, long rows, long N) {
 
 }  // namespace
 
+// Workspace of the middle-size kernels' K splits (hn_mid.hip), after the counter
+// region.
+extern "C" long hn_mid_part_bytes(int mats, long M, long N, long K);
+
 // Bytes of workspace hn_int4_linear / hn_int4_gate_up_silu / hn_expert_mlp_int4 /
 // hn_grouped_expert_mlp_int4 need.  kind: 0 linear (M,N,K), 1 gate_up (M,N=I,K=H),
 // 2 expert mlp (M=T, N=H, K=I), 3 grouped (M=rows=T*k, N=H, K=I, E).
@@ -555,7 +560,9 @@ extern "C" long hn_skinny_workspace_bytes(int kind, long M, long N, long K, long
   if (kind == 0 || kind == 1) {
     const int mats = kind == 0 ? 1 : 2;
     const Plan p = make_plan(r, (int)K, mats);
-    return (long)(ctr_bytes(hn_cdiv(N, kTileN)) + part_bytes(p.ks, mats, r, N));
+    const size_t a = part_bytes(p.ks, mats, r, N);
+    const size_t b = r > kStreamMaxRows ? (size_t)hn_mid_part_bytes(mats, r, N, K) : 0;
+    return (long)(ctr_bytes(hn_cdiv(N, kTileN)) + (a > b ? a : b));
   }
   // kind 2: expert MLP, N = H, K = I.  kind 3: grouped over E experts, M = all rows.
   const long H = N, I = K;
@@ -567,6 +574,11 @@ extern "C" long hn_skinny_workspace_bytes(int kind, long M, long N, long K, long
   const size_t a = part_bytes(pg.ks, 2, prow, I);
   const size_t b = part_bytes(pd.ks, 1, prow, H);
   size_t m = a > b ? a : b;
+  if (kind == 2 && r > kStreamMaxRows) {
+    const long c = hn_mid_part_bytes(2, r, I, H), d = hn_mid_part_bytes(1, r, H, I);
+    const size_t e = (size_t)(c > d ? c : d);
+    m = m > e ? m : e;
+  }
   if (kind == 3) {  // hn_moe_experts_decode: fp32 K-slice partials of the down projection
     const size_t c = (size_t)kHnDownSplit * prow * H * 4;
     m = m > c ? m : c;
@@ -613,6 +625,19 @@ extern "C" int hn_moe_unpermute_split4_impl(const float* part, long ks_stride, c
                                             const void* shared, long ld_sh, void* out,
                                             long ld_o, long H, void* stream);
 
+// Kernels for a middle number of rows per matrix (hn_mid.hip): same return
+// convention.
+extern "C" int hn_mid_linear_impl(int mats, const void* x, long ld_x, const void* q0,
+                                  const void* s0, const void* q1, const void* s1, long ld_q,
+                                  long ld_s, void* out, long ld_o, long M, long N, long K,
+                                  long group, void* work, long work_bytes, void* stream);
+extern "C" int hn_mid_grouped_impl(int phase, const void* x, long ld_x, const void* table,
+                                   const int* active, const int* n_active, const int* offsets,
+                                   long E, long rows, long H, long I, long group, void* out,
+                                   long ld_o, float* part, int ks, void* stream, int dry_run);
+extern "C" int hn_mid_reduce_impl(const float* part, int ks, long rows, long N, void* out,
+                                  long ld_o, void* stream);
+
 // Prefill GEMM kernels (hn_gemm.hip): same return convention.
 extern "C" int hn_gemm_linear_impl(int mats, const void* x, long ld_x, const void* q0,
                                    const void* s0, const void* q1, const void* s1, long ld_q,
@@ -628,19 +653,46 @@ extern "C" long hn_gemm_workspace_bytes();
 // 1 = split-K kernels only.  Per calling thread (a switch in one thread never
 // changes another thread's calls); for A/B measurement and tests.
 static thread_local int g_decode_path = 0;
-constexpr long kStreamMaxRows = 16;
 
-// Whether the streaming kernels take a grouped decode launch.  They stage at
-// most 8 tokens of an expert per pass over its weights, so an expert with more
-// rows streams its weights once per 8; they are used up to 16 rows per expert,
-// or up to 64 when the average over the experts is at most 8 (few rows per
-// expert: GLM-4.5-Air's 128 experts x top-8; 64 tokens over 8 experts at top-1
-// pass over each expert's weights about 1.4 times on average).
-// The streaming kernels take a grouped launch when every expert's rows fit
-// one pass (<= 16), or when the rows average at most 16 per expert (passes
-// of 8 or 16 tokens; the decoder's 64-token batches at top-1 and top-2).
+// Which kernels take a grouped launch of group 128.  Up to 16 rows per expert the
+// streaming kernels do, in one pass over the weights; past that by the average:
+//  * up to 10 rows per expert the streaming kernels (passes of 8 or 16 tokens of
+//    whole K, at most 64 rows): us gate/up + down, 8 experts of 4096 x 14336,
+//    8 rows each 95 + 50 against 111 + 61 by the middle-size kernels; 12 rows
+//    113 + 67 against 113 + 62;
+//  * up to 128 rows the middle-size kernels (hn_mid.hip): 24 rows each 129 + 66
+//    against 241 + 126 by the prefill GEMM, 128 rows 310 + 155 against 319 + 163;
+//    128 experts of 4096 x 1408, 32 rows 196 + 122 against 367 + 237.  Above 64
+//    rows for one expert they also take the smaller averages, where the
+//    streaming kernels' bound on an expert's rows does not hold;
+//  * above, the prefill GEMM (192 rows each 410 + 230 against 447 + 233).
+constexpr long kStreamAvgRows = 10, kMidAvgRows = 128;
 static bool stream_rows_ok(long max_rows, long rows, long E) {
   return max_rows <= kStreamMaxRows || (max_rows <= kMaxRows && rows <= 16 * E);
+}
+
+// K slices of the middle-size kernels' down projection: whole where a row's
+// scales fit their LDS copy, else the split the unpermute sums (0: neither).
+static int mid_down_split(long E, long rows, long H, long I, long group) {
+  static float dummy;
+  if (hn_mid_grouped_impl(1, nullptr, I, nullptr, nullptr, nullptr, nullptr, E, rows, H, I, group,
+                          nullptr, H, nullptr, 1, nullptr, 1) == 0)
+    return 1;
+  return hn_mid_grouped_impl(1, nullptr, I, nullptr, nullptr, nullptr, nullptr, E, rows, H, I,
+                             group, nullptr, H, &dummy, kHnDownSplit, nullptr, 1) == 0
+             ? kHnDownSplit : 0;
+}
+
+static bool mid_grouped_ok(long E, long max_rows, long rows, long H, long I, long group) {
+  if (g_decode_path != 0 || max_rows <= kStreamMaxRows || rows > kMidAvgRows * E) return false;
+  if (max_rows <= kMaxRows && rows <= kStreamAvgRows * E) return false;
+  return hn_mid_grouped_impl(0, nullptr, H, nullptr, nullptr, nullptr, nullptr, E, rows, H, I,
+                             group, nullptr, I, nullptr, 1, nullptr, 1) == 0 &&
+         mid_down_split(E, rows, H, I, group) != 0;
+}
+
+static long mid_down_bytes(long rows, long H) {
+  return (long)kCtrRegion + (long)kHnDownSplit * rows * H * 4;
 }
 
 extern "C" int hn_set_decode_path(int path) {
@@ -671,6 +723,11 @@ static int run_single(int mats, const void* x, long ld_x, W4Mat w0, W4Mat w1, vo
                "%s: one weight matrix must stay below 2 GiB - 16 B", who);
   if (M == 0 || N == 0) return 0;
   const bool premul = (group % 128) != 0;
+  if (g_decode_path == 0 && M > kStreamMaxRows) {
+    const int rc = hn_mid_linear_impl(mats, x, ld_x, w0.q, w0.s, w1.q, w1.s, w0.ld_q, w0.ld_s, out,
+                                      ld_o, M, N, K, group, ws, ws_size, s);
+    if (rc != HN_NOT_HANDLED) return rc;
+  }
   if (M > kMaxRows) {
     const int rc = hn_gemm_linear_impl(mats, x, ld_x, w0.q, w0.s, w1.q, w1.s, w0.ld_q, w0.ld_s,
                                        out, ld_o, M, N, K, group, ws, ws_size, s);
@@ -806,6 +863,19 @@ extern "C" int hn_grouped_expert_mlp_int4(const void* x_perm, const void* table,
   HN_ARG_CHECK(I * (H / 2) < 0x7ffffff0L && I * (H / group) * 2 < 0x7ffffff0L,
                "%s: one weight matrix must stay below 2 GiB - 16 B", who);
   if (max_rows_per_expert == 0 || rows == 0) return 0;
+  if (mid_grouped_ok(E, max_rows_per_expert, rows, H, I, group)) {
+    const int ks = mid_down_split(E, rows, H, I, group);
+    if (ks == 1 || (work && aligned16(work) && work_bytes >= mid_down_bytes(rows, H))) {
+      float* part = ks == 1 ? nullptr : (float*)((char*)work + kCtrRegion);
+      int rc = hn_mid_grouped_impl(0, x_perm, H, table, active, n_active, offsets, E, rows, H, I,
+                                   group, h_ws, I, nullptr, 1, stream, 0);
+      if (rc == 0)
+        rc = hn_mid_grouped_impl(1, h_ws, I, table, active, n_active, offsets, E, rows, H, I,
+                                 group, y_perm, H, part, ks, stream, 0);
+      if (rc == 0 && part) rc = hn_mid_reduce_impl(part, ks, rows, H, y_perm, H, stream);
+      return rc;
+    }
+  }
   if (max_rows_per_expert > kMaxRows) {
     // prefill: the grouped MFMA GEMM (a workspace of hn_gemm_workspace_bytes
     // enables its stream-K split; without one whole tiles go round-robin)
@@ -916,9 +986,11 @@ extern "C" int hn_grouped_expert_phase_int4(int phase, const void* x_perm, const
   return rc;
 }
 
-// Whether hn_moe_experts_decode takes the streaming path with the K-split down
-// projection for these sizes (the launches' own dry runs).
+// Whether hn_moe_experts_decode runs the down projection in K slices for these
+// sizes, by the streaming or the middle-size kernels (their own dry runs).
 static bool experts_split_ok(long E, long max_rows, long rows, long H, long I, long group) {
+  if (rows > 0 && mid_grouped_ok(E, max_rows, rows, H, I, group))
+    return mid_down_split(E, rows, H, I, group) == kHnDownSplit;
   return rows > 0 && max_rows > 0 && stream_rows_ok(max_rows, rows, E) && g_decode_path == 0 &&
          group % 128 == 0 && H % 128 == 0 && I % 128 == 0 &&
          hn_stream_grouped_impl(0, nullptr, H, nullptr, nullptr, nullptr, nullptr, E, max_rows,
@@ -952,8 +1024,12 @@ extern "C" int hn_moe_experts_decode(const void* x_perm, const void* table, cons
                "%s: out rows must be 16-byte aligned", who);
   hipStream_t s = (hipStream_t)stream;
   if (!out && rows == 0) return 0;  // no rows: no partials to leave
+  // (the middle-size kernels' slices also need the workspace, which the prefill
+  // GEMM behind them can do without)
+  const bool mid = mid_grouped_ok(E, max_rows_per_expert, rows, H, I, group);
   const bool split = experts_split_ok(E, max_rows_per_expert, rows, H, I, group) &&
-                     aligned16(x_perm) && aligned16(h_ws);
+                     aligned16(x_perm) && aligned16(h_ws) &&
+                     (!mid || !out || (work && work_bytes >= mid_down_bytes(rows, H)));
   HN_ARG_CHECK(out || (split && !shared),
                "%s: out NULL (partials left for the caller) needs the streaming path with the "
                "K-split down projection (hn_moe_experts_decode_split_check) and no shared "
@@ -961,15 +1037,24 @@ extern "C" int hn_moe_experts_decode(const void* x_perm, const void* table, cons
   if (split) {
     const long tmax = hn_cdiv(I, kTileN) > hn_cdiv(H, kTileN) ? hn_cdiv(I, kTileN)
                                                               : hn_cdiv(H, kTileN);
-    const long need = hn_skinny_workspace_bytes(3, rows, H, I, E);
+    const long need = mid ? mid_down_bytes(rows, H) : hn_skinny_workspace_bytes(3, rows, H, I, E);
     HN_ARG_CHECK(work && work_bytes >= need, "%s: workspace too small (%ld < %ld)", who,
                  work_bytes, need);
     float* part = (float*)((char*)work + ctr_bytes(E * tmax));
-    int rc = hn_stream_grouped_impl(0, x_perm, H, table, active, n_active, offsets, E,
-                                    max_rows_per_expert, rows, H, I, group, h_ws, I, s, 0);
-    if (rc == 0)
-      rc = hn_stream_down_split_impl(h_ws, table, active, n_active, offsets, E,
-                                     max_rows_per_expert, rows, H, I, group, part, s, 0);
+    int rc;
+    if (mid) {
+      rc = hn_mid_grouped_impl(0, x_perm, H, table, active, n_active, offsets, E, rows, H, I, group,
+                               h_ws, I, nullptr, 1, stream, 0);
+      if (rc == 0)
+        rc = hn_mid_grouped_impl(1, h_ws, I, table, active, n_active, offsets, E, rows, H, I, group,
+                                 nullptr, H, part, kHnDownSplit, stream, 0);
+    } else {
+      rc = hn_stream_grouped_impl(0, x_perm, H, table, active, n_active, offsets, E,
+                                  max_rows_per_expert, rows, H, I, group, h_ws, I, s, 0);
+      if (rc == 0)
+        rc = hn_stream_down_split_impl(h_ws, table, active, n_active, offsets, E,
+                                       max_rows_per_expert, rows, H, I, group, part, s, 0);
+    }
     if (rc == 0 && out)
       rc = hn_moe_unpermute_split4_impl(part, rows * H, inv, idx, w, T, k, shared, ld_sh, out,
                                         ld_o, H, stream);

@@ -315,24 +315,16 @@ def moe_dispatch(r: Routed, table: ExpertTable,
     assert fold is None or (shared is None and T <= _lib.DECODE_MAX_ROWS), \
         "moe_dispatch: fold needs the decode path and no shared expert"
     out = torch.empty((T, H), dtype=torch.float16, device=dev) if fold is None else None
-    if T <= _lib.DECODE_MAX_ROWS:
-        # decode: both expert phases and the unpermute (split down projection)
-        work = _lib.skinny_workspace(3, n, H, I, E, dev)
-        _lib.call("hn_moe_experts_decode", _lib.ptr(r.x_perm), _lib.ptr(table.dev),
-                  _lib.ptr(r.active), _lib.ptr(r.n_active), _lib.ptr(r.offsets), E, T, n, H, I,
-                  g, _lib.ptr(h_ws), _lib.ptr(y_perm), _lib.ptr(r.inv), _lib.ptr(r.idx),
-                  _lib.ptr(r.w), T, k, _lib.ptr(sh), H if sh is None else sh.stride(0),
-                  _lib.ptr(out), H, _lib.ptr(work), work.numel(), st)
-        return out if fold is None else _unpermute_add_rmsnorm(work, r, H, I, fold)
-    work = _lib.gemm_workspace(dev)  # stream-K split of the prefill GEMM
-    _lib.call("hn_grouped_expert_mlp_int4", _lib.ptr(r.x_perm), _lib.ptr(table.dev),
+    # both expert phases and the unpermute (the down projection in K slices
+    # where the decode and middle-size kernels run it so)
+    work = (_lib.skinny_workspace(3, n, H, I, E, dev) if T <= _lib.DECODE_MAX_ROWS
+            else _lib.gemm_workspace(dev))
+    _lib.call("hn_moe_experts_decode", _lib.ptr(r.x_perm), _lib.ptr(table.dev),
               _lib.ptr(r.active), _lib.ptr(r.n_active), _lib.ptr(r.offsets), E, T, n, H, I, g,
-              _lib.ptr(h_ws), _lib.ptr(y_perm), _lib.ptr(work),
-              0 if work is None else work.numel(), st)
-    _lib.call("hn_moe_unpermute", _lib.ptr(y_perm), H, _lib.ptr(r.inv), _lib.ptr(r.idx),
-              _lib.ptr(r.w), T, k, _lib.ptr(sh), H if sh is None else sh.stride(0), _lib.ptr(out),
-              H, H, st)
-    return out
+              _lib.ptr(h_ws), _lib.ptr(y_perm), _lib.ptr(r.inv), _lib.ptr(r.idx), _lib.ptr(r.w),
+              T, k, _lib.ptr(sh), H if sh is None else sh.stride(0), _lib.ptr(out), H,
+              _lib.ptr(work), work.numel(), st)
+    return out if fold is None else _unpermute_add_rmsnorm(work, r, H, I, fold)
 
 
 def moe_experts_forward(hidden: torch.Tensor, idx: torch.Tensor, w: torch.Tensor,

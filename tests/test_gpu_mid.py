@@ -1,0 +1,126 @@
+"""The kernels for a middle number of rows per weight matrix (csrc/hn_mid.hip)
+against float64 products of the dequantised weights, at the edges of their tiles
+(32 and 64 tokens, 256 weight rows), K splits (even, uneven, none) and group
+sizes, single and grouped.
+
+Tolerance: the repository's bar for fp16 matrix outputs, 1e-2 + 2e-3 |ref|: one
+fp16 rounding of the result (2^-11 relative), for groups under 128 one more per
+weight (2^-11, averaging out over K), fp32 sums.  For the SwiGLU the two
+projections round to fp16 first (1e-2 covers 2^-11 of either at these sizes)."""
+import pytest
+import torch
+
+from hydranet_amd import _lib
+from hydranet_amd.kernels import int4_gemm as g
+from hydranet_amd.model import moe
+
+pytestmark = pytest.mark.gpu
+
+
+def _weight(n, k, group, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    w = torch.randn(n, k, generator=gen, device="cuda").mul_(0.02).half()
+    return g.quantize_int4(w, group)
+
+
+def _deq(p, s):
+    n, k = p.shape[0], 2 * p.shape[1]
+    code = torch.stack((p & 15, p >> 4), 2).view(n, k).double() - 8
+    return (code.view(n, s.shape[1], -1) * s.double().unsqueeze(2)).view(n, k)
+
+
+def _x(m, k, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(m, k, generator=gen, device="cuda").half()
+
+
+def _close(y, ref):
+    err = (y.double() - ref).abs() - 2e-3 * ref.abs()
+    assert bool(torch.isfinite(y).all()) and err.max().item() <= 1e-2, err.max().item()
+
+
+@pytest.mark.parametrize("m,n,k,group", [
+    (17, 4096, 4096, 128), (32, 256, 128, 128), (33, 272, 256, 128), (64, 6144, 4096, 128),
+    (65, 100, 1408, 128), (40, 1408, 1408, 128), (200, 4096, 14336, 128), (333, 4096, 4096, 64),
+    (48, 1030, 640, 64), (19, 512, 4096, 32), (512, 1000, 2048, 32), (24, 4094, 4096, 128),
+])
+def test_linear(m, n, k, group):
+    print(f"[mid] linear m={m} n={n} k={k} group={group}", flush=True)
+    p, s = _weight(n, k, group, m + n)
+    x = _x(m, k, m)
+    y = g.int4_linear(x, p, s, group)
+    _close(y, x.double() @ _deq(p, s).t())
+    assert torch.equal(y, g.int4_linear(x, p, s, group))  # sums in split order: repeatable
+
+
+@pytest.mark.parametrize("t,h,i,group", [(17, 512, 768, 128), (37, 4096, 14336, 128),
+                                         (64, 1024, 1408, 64), (130, 640, 2048, 128)])
+def test_expert(t, h, i, group):
+    print(f"[mid] expert t={t} h={h} i={i} group={group}", flush=True)
+    ws = [_weight(a, b, group, 7 + j) for j, (a, b) in enumerate(((i, h), (i, h), (h, i)))]
+    x = _x(t, h, t)
+    y = g.expert_mlp_int4_fused(x, *[v for w in ws for v in w], group_size=group)
+    dg, du, dd = (_deq(*w) for w in ws)
+    hid = torch.nn.functional.silu(x.double() @ dg.t()) * (x.double() @ du.t())
+    _close(y, hid @ dd.t())
+
+
+def _layer(e, h, i, seed):
+    from hydranet_amd.preprocess.synthetic import make_expert_slot
+    return [make_expert_slot(seed + j, h, i, 128, slot_idx=j) for j in range(e)]
+
+
+@pytest.mark.parametrize("e,h,i,tokens,k", [
+    (8, 512, 2048, 70, 2),     # down in one piece, over 64 tokens
+    (8, 512, 6144, 60, 2),     # 48 stages: the down projection in K slices
+    (4, 512, 2048, 300, 2),    # 150 rows per expert: past these kernels, the prefill GEMM
+    (16, 256, 1408, 90, 4),    # ragged I
+])
+def test_experts_uneven(e, h, i, tokens, k):
+    """Experts with no rows, one row, and most of the rows."""
+    print(f"[mid] experts e={e} h={h} i={i} tokens={tokens} k={k}", flush=True)
+    slots = _layer(e, h, i, 11)
+    table = moe.ExpertTable.from_slots(slots)
+    gen = torch.Generator().manual_seed(e + tokens)
+    p = torch.tensor([0.0, 1e-4] + [2.0 ** -j for j in range(e - 2)]) + 1e-9
+    idx = torch.multinomial(p.expand(tokens, e), k, generator=gen)
+    idx[idx == 0] = e - 1                      # expert 0: no rows (duplicates are allowed)
+    w = torch.rand(tokens, k, generator=gen).half()
+    x = _x(tokens, h, 3)
+    out = moe.moe_experts_forward(x, idx.int().cuda(), w.cuda(), table)
+    ref = torch.zeros(tokens, h, dtype=torch.float64, device="cuda")
+    for j in range(e):
+        rows, slot = (idx == j).nonzero(as_tuple=True)
+        if len(rows):
+            s = slots[j]
+            xe = x[rows.cuda()].double()
+            hid = torch.nn.functional.silu(xe @ _deq(s.gate_packed, s.gate_scales).t()) * (
+                xe @ _deq(s.up_packed, s.up_scales).t())
+            y = hid @ _deq(s.down_packed, s.down_scales).t()
+            ref.index_add_(0, rows.cuda(), y * w[rows, slot].double().cuda().unsqueeze(1))
+    # k roundings of the weighted rows and of their fp16 sum beside the products' own
+    _close(out / k, ref / k)
+
+
+@pytest.mark.parametrize("t,k,i", [(96, 2, 2048), (96, 2, 6144), (33, 4, 2048)])
+def test_layer_graph_replay(t, k, i):
+    """The layer's launches captured once and replayed: every replay as the eager run."""
+    print(f"[mid] graph t={t} k={k} i={i}", flush=True)
+    layer = moe.MixtralMoELayer(512, 8, k, slots=_layer(8, 512, i, 5)).cuda().half().eval()
+    x = _x(t, 512, 9).view(1, t, 512)
+    with torch.no_grad():
+        want = layer(x, top_k=k).clone()
+        st = torch.cuda.Stream()
+        st.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(st):
+            layer(x, top_k=k)
+        torch.cuda.current_stream().wait_stream(st)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = layer(x, top_k=k)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+            assert torch.equal(layer(x, top_k=k), want)
