@@ -39,6 +39,8 @@ SIGNATURES: dict[str, list] = {
     "hn_moe_unpermute": [P, L, P, P, P, L, L, P, L, P, L, L, P],
     "hn_add_rmsnorm": [P, L, P, L, P, L, P, P, L, L, L, F, P],
     "hn_add_rmsnorm_router": [P, L, P, L, P, L, P, P, L, L, L, F, P, L, L, P, P],
+    "hn_attn_prefill_workspace_bytes": [L, L, L],
+    "hn_attn_prefill": [P, P, P, L, L, L, L, L, L, L, P, L, F, P, L, P, P],
     "hn_attn_softmax": [P, L, P, L, L, L, L, F, P, L, P],
     "hn_attn_decode": [P, P, P, L, L, L, L, L, L, P, F, P, L, P],
     "hn_unpermute_add_rmsnorm": [P, L, L, P, P, P, L, L, P, L, P, L, P, P, L, L, F, P],
@@ -72,7 +74,8 @@ SIGNATURES: dict[str, list] = {
 ROUTE_MAX_LOGITS = 8192   # T * E
 ROUTE_MAX_ASSIGN = 1024   # T * k
 
-RESTYPES = {"hn_skinny_workspace_bytes": ctypes.c_long, "hn_gemm_workspace_bytes": ctypes.c_long,
+RESTYPES = {"hn_skinny_workspace_bytes": ctypes.c_long,
+            "hn_attn_prefill_workspace_bytes": ctypes.c_long, "hn_gemm_workspace_bytes": ctypes.c_long,
             "hn_moe_decode_layer_partials": ctypes.c_long}
 
 # Tokens per weight matrix up to which the decode (skinny / streaming) kernels

@@ -135,8 +135,9 @@ class Attention(nn.Module):
         self.k_proj = nn.Linear(H, self.nkv * self.hd, bias=False)
         self.v_proj = nn.Linear(H, self.nkv * self.hd, bias=False)
         self.o_proj = nn.Linear(self.nh * self.hd, H, bias=False)
-        # one-token steps on the GPU: attention in one launch (hn_attn_decode)
-        # where its shape limits allow; False keeps the two products
+        # on the GPU, attention in one launch (hn_attn_decode for one-token
+        # steps, hn_attn_prefill for more) where its shape limits allow; False
+        # keeps the two products
         self.decode_kernel = True
 
     def _decode_fits(self, x: torch.Tensor, S: int, cache: "KVCache", kv_len: int,
@@ -146,6 +147,26 @@ class Attention(nn.Module):
                 and cache.max_len % 8 == 0 and cache.max_len >= -(-kv_len // 8) * 8
                 and (mask is None or (mask.dtype == torch.float16 and mask.numel() == kv_len
                                       and mask.is_contiguous())))
+
+    def _prefill_fits(self, x: torch.Tensor, S: int, cache: "KVCache", kv_len: int,
+                      mask: Optional[torch.Tensor]) -> bool:
+        """The one-kernel form walks a workgroup's positions one tile of 64
+        after the other (about 1.9 us each); the two products spread a long
+        past over the chip.  Their times cross where there are about as many
+        workgroups as tiles (B, S, past: one kernel / products, us, whole
+        module): 1, 32, 1000 (8 and 17): 82 / 69; 2, 64, 2000 (32 and 33): 134 /
+        137; 1, 128, 4000 (32 and 65): 203 / 186; 1, 256, 4000 (64 and 67): 219 /
+        334; 8, 333, 0 (96 x 8 and 6): 263 / 421."""
+        rep = self.nh // self.nkv
+        rows = S * rep if S < 128 else S  # see hn_attn_prefill: heads share a tile below 128
+        wgs = x.shape[0] * self.nh * S // rows * -(-rows // 128)
+        return (self.decode_kernel and x.is_cuda and S > 1 and self.hd == 128
+                and 8 * wgs >= 7 * -(-kv_len // 64)
+                and cache.max_len % 8 == 0 and 1 <= kv_len <= cache.max_len < 1 << 22
+                and rep * S < 1 << 22
+                and (mask is None or (mask.dtype == torch.float16 and mask.is_cuda
+                                      and tuple(mask.shape) == (S, kv_len)
+                                      and mask.stride(1) == 1 and mask.stride(0) >= kv_len)))
 
     def _qkv(self, x2: torch.Tensor) -> torch.Tensor:
         """q, k and v projections of x2 [rows, H] as one product: the fp16
@@ -227,6 +248,19 @@ class Attention(nn.Module):
             _lib.call("hn_attn_decode", _lib.ptr(qg), _lib.ptr(cache.kt[layer]),
                       _lib.ptr(cache.v[layer]), cache.max_len, B, nkv, rep, hd, kv_len,
                       _lib.ptr(mask), inv, _lib.ptr(o), o.stride(0), _lib.stream(x.device))
+            return self.o_proj(o.view(B, S, nh * hd))
+        if self._prefill_fits(x, S, cache, kv_len, mask):
+            from .. import _lib
+            o = torch.empty((B * S, nh * hd), dtype=x.dtype, device=x.device)
+            work = None
+            if mask is not None:
+                work = torch.empty(_lib.lib().hn_attn_prefill_workspace_bytes(S, rep, kv_len),
+                                   dtype=torch.uint8, device=x.device)
+            inv = float(np.float32(1.0) / np.float32(math.sqrt(hd)))
+            _lib.call("hn_attn_prefill", _lib.ptr(qg), _lib.ptr(cache.kt[layer]),
+                      _lib.ptr(cache.v[layer]), cache.max_len, B, nkv, rep, hd, S, kv_len,
+                      _lib.ptr(mask), 0 if mask is None else mask.stride(0), inv, _lib.ptr(o),
+                      o.stride(0), _lib.ptr(work), _lib.stream(x.device))
             return self.o_proj(o.view(B, S, nh * hd))
         kt, vv = cache.get(layer, kv_len)
         scores = torch.matmul(qg, kt)  # [B, nkv, rep * S, kv_len]

@@ -401,6 +401,27 @@ int hn_attn_decode_rope(const void* qkv, long ld_qkv, const float* cos_t, const 
                         const long* pos, void* kt, void* v, long max_len, long B, long nkv,
                         long rep, long hd, long L, const void* mask, float inv_scale, void* out,
                         long ld_o, void* stream);
+
+/* hn_attn_prefill: grouped-query attention of S query tokens per sequence
+ *   over the KV cache's first L positions, scores, mask, softmax and value
+ *   product in one pass (the reference's Attention, model/mixtral.py:193-207,
+ *   for more than one token; the scores are never written).  q [B][nkv][rep]
+ *   [S][hd] fp16 (hn_rope_append's q_out), kt [B][nkv][hd][max_len], v [B]
+ *   [nkv][max_len][hd], mask [S, L] fp16 (row stride ld_m, added to the
+ *   scores) or NULL; out[(b * S + s) * ld_o + (g * rep + r) * hd + d].  fp32
+ *   scores, maximum, exponentials and sums, probabilities rounded to fp16 for
+ *   the product; where a mask holds values other than 0 and -inf the scores
+ *   are rounded to fp16, scaled, rounded, masked and rounded as hn_attn_softmax
+ *   rounds them.  Blocks of 32 rows x 64 positions whose mask is all -inf are
+ *   not computed, so a NaN or infinity there does not reach the rows; a row
+ *   with every position at -inf gives NaN.  hd 128, max_len a multiple of 8,
+ *   rep * S < 2^22, 16-byte aligned operands (mask: any), ld_o a multiple of 8.
+ *   work: hn_attn_prefill_workspace_bytes(S, rep, L) bytes (16-byte aligned,
+ *   any contents) with a mask, unused without. */
+long hn_attn_prefill_workspace_bytes(long S, long rep, long L);
+int hn_attn_prefill(const void* q, const void* kt, const void* v, long max_len, long B, long nkv,
+                    long rep, long hd, long S, long L, const void* mask, long ld_m,
+                    float inv_scale, void* out, long ld_o, void* work, void* stream);
 int hn_rope_append(const void* q, long ld_q, const void* k, long ld_k, const void* v, long ld_v,
                    const float* cos_t, const float* sin_t, const long* pos, long B, long S,
                    long nh, long nkv, long hd, void* q_out, void* kt, void* vc, long max_len,
