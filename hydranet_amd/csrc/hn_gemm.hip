@@ -21,8 +21,8 @@
 //    exactly one wave per tile.
 //  * Every load of the K loop goes HBM -> LDS directly (buffer_load ... lds,
 //    with explicit waits), three LDS stages of 64 k:
-//    activations (XOR-swizzled rows so A-fragment reads are conflict-free),
-//    packed weights and the dwords holding the scales.
+//    activations (XOR-swizzled rows so A-fragment reads are conflict-free) and
+//    packed weights; scales by runs of 8 groups.
 //  * Each k-step's A fragments and unpacked weights are double-buffered: step
 //    s + 1's LDS reads and unpack are issued ahead of / under step s's MFMAs.
 //    A packed dword becomes eight fp16 weights in k order: a byte broadcast
@@ -142,11 +142,6 @@ __device__ __forceinline__ void dma_b128(__amdgpu_buffer_rsrc_t r, uint32_t voff
                                            voff, __builtin_amdgcn_readfirstlane(soff), 0, 0);
 }
 
-__device__ __forceinline__ void dma_b32(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t lds) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds_ptr(__builtin_amdgcn_readfirstlane(lds)), 4,
-                                           voff, 0, 0, 0);
-}
-
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
@@ -192,17 +187,31 @@ constexpr int kNST = 3;            // LDS stages
 
 // LDS stage (bytes): activations [256 rows][kChunks chunks of 16 B], chunk c of
 // row r at slot c ^ key(r), so the 8 or 16 rows an A-fragment read serves per
-// LDS cycle hit distinct banks; packed weights [wave][block][d][lane] 16 B;
-// scale dwords [wave][block][lane] 4 B.
+// LDS cycle hit distinct banks; packed weights [wave][block][d][lane] 16 B.
 struct Stage {
   static constexpr int kA = 0;
   static constexpr int kB = kBMMax * kChunks * 16;
-  static constexpr int kS = kB + kWaves * kBlk * kKSM * 1024;
-  static constexpr int kSize = kS + kWaves * kBlk * 256;
+  static constexpr int kSize = kB + kWaves * kBlk * kKSM * 1024;
 };
-// activation loads per lane for a tile of NRB row blocks; loads per stage
+
+// Scales, outside the stages: runs of kScRun groups, two slots in turn, each
+// [wave][block][half run][32 rows] 16 B: lane l's load brings 16 bytes holding
+// the run's groups 4 (l / 32) .. + 3 of row l % 32.  A run lasts kScRun group /
+// kKS stages (four at the least), so the two slots are never both needed by
+// loads in flight and reads to come.
+// (A gather of 32 rows costs the vector memory path about as much for a dword
+// as for 16 bytes, 65 cycles, so loading each stage's scale dwords anew took 520
+// cycles of the CU's path per stage, next to 1350 for activations and weights
+// and 2048 for the stage's MFMAs.  4096 rows over eight Mixtral experts on
+// MI355X, per-stage dwords and runs: gate/up 991 -> 979 us, down 511 -> 483 us;
+// the layer of 2048 tokens 1725 -> 1700 us.)
+constexpr int kScRun = 8;
+constexpr int kScSlot = kWaves * kBlk * 1024;  // bytes
+constexpr int kLdsBytes = kNST * Stage::kSize + 2 * kScSlot;
+// activation loads per lane for a tile of NRB row blocks; loads per stage (the
+// first stage of a scale run issues kBlk more)
 template <int NRB> constexpr int a_loads() { return kChunks * 32 * NRB / (kWaves * 64); }
-template <int NRB> constexpr int loads_per_stage() { return a_loads<NRB>() + kBlk * kKSM + kBlk; }
+template <int NRB> constexpr int loads_per_stage() { return a_loads<NRB>() + kBlk * kKSM; }
 constexpr int kALoadsMax = a_loads<kRBMax>();
 
 __device__ __forceinline__ int akey(int r) {
@@ -217,10 +226,10 @@ struct TileLoads {
   const void* px; int nx;             // activation rows of the tile, bytes
   const void* pq[kBlk];               // packed weights of each block's matrix
   const void* ps[kBlk];               // scales
-  int nq, ns;                         // bytes of one packed / scale matrix
+  int nq, ns;                         // bytes of one packed / scale matrix (ns: whole dwords)
   uint32_t va[kALoadsMax];            // activation chunk offsets (first a_loads<NRB>)
   uint32_t vq[kBlk];                  // weight byte offset of (lane's row, lane's 16 B)
-  uint32_t vs[kBlk];                  // scale byte offset of (lane's row, lane's k)
+  uint32_t vs[kBlk];                  // scale byte offset of the lane's row
   int group;
 };
 
@@ -236,18 +245,34 @@ __device__ __forceinline__ uint32_t a_offset(int j, int wave, int lane, int rows
   return (uint32_t)((min(r, rows - 1) * (int)ld_x + 8 * c) * 2);
 }
 
-// Issue stage t's loads into the LDS stage at byte address st.  Weights: per
-// block kKSM loads; load d brings lane l's 16 bytes at 16 kKSM (l / 32) + 16 d
-// of row (l % 32)'s 32 kKSM bytes of the stage.  Scales: the dword holding the
-// lane's scale.  With real false the same loads go out against empty buffer
-// ranges: they read nothing from memory (out of range), write zeros into a
-// stage no one reads, and keep the count of loads per stage fixed, so the
-// K loop's waits are the same at every stage (no branch in the loop).
+// Byte offset of the 16 bytes holding groups g .. g + 3 (g a multiple of 4) of
+// the row whose scales start at byte row: the dword of group g, moved back
+// where 16 bytes would end past the matrix.
+__device__ __forceinline__ uint32_t scale_src(const TileLoads& tl, uint32_t row, int g) {
+  return min((row + 2 * g) & ~3u, (uint32_t)tl.ns - 16);
+}
+
+// Issue stage t's loads into the LDS stage at byte address st, and those of
+// the scale run (slots at sc0) that starts with it.  grp: scale group of the
+// stage's first k.  Weights: per block kKSM loads; load d brings lane l's 16
+// bytes at 16 kKSM (l / 32) + 16 d of row (l % 32)'s 32 kKSM bytes of the
+// stage.  With real false the same activation and weight loads go out against
+// empty buffer ranges: they read nothing from memory (out of range), write
+// zeros into a stage no one reads, and keep the count of loads per stage
+// fixed, so the K loop's waits are the same at every stage.  A run's loads are
+// the stage's first: a wait that leaves loads_per_stage in flight is then right
+// with them too (it waits for them as well).
 template <int NRB>
-__device__ __forceinline__ void issue_stage(const TileLoads& tl, int t, uint32_t st, int wave,
-                                            bool real) {
+__device__ __forceinline__ void issue_stage(const TileLoads& tl, int t, int grp, uint32_t st,
+                                            uint32_t sc0, int wave, int h, bool real) {
   using L = Stage;
   constexpr int NA = a_loads<NRB>();
+  if (real && grp % kScRun == 0 && grp * tl.group == kKS * t) {  // uniform
+#pragma unroll
+    for (int b = 0; b < kBlk; ++b)
+      dma_b128(rsrc(tl.ps[b], tl.ns), scale_src(tl, tl.vs[b], grp + 4 * h), 0,
+               sc0 + (grp / kScRun & 1) * kScSlot + (wave * kBlk + b) * 1024);
+  }
   {
     const __amdgpu_buffer_rsrc_t r = rsrc(tl.px, real ? tl.nx : 0);
 #pragma unroll
@@ -262,11 +287,6 @@ __device__ __forceinline__ void issue_stage(const TileLoads& tl, int t, uint32_t
       dma_b128(r, tl.vq[b] + 16 * d, kKS / 2 * t,
                st + L::kB + ((wave * kBlk + b) * kKSM + d) * 1024);
   }
-  const uint32_t soff = 2 * ((kKS * t) / tl.group);
-#pragma unroll
-  for (int b = 0; b < kBlk; ++b)
-    dma_b32(rsrc(tl.ps[b], real ? tl.ns : 0), (tl.vs[b] + soff) & ~3u,
-            st + L::kS + (wave * kBlk + b) * 256);
 }
 
 // Unpack constants (gfx9 VOP3 takes no literals): mask in an SGPR, the rest
@@ -326,13 +346,15 @@ __device__ __forceinline__ void read_a(Ops& o, int buf, uint32_t st, int s, int 
     o.af[buf][rb] = lds_read<half8_t>(base + rb * 32 * kChunks * 16);
 }
 
-// Weights + scales of the stage at st (stage number t); half-word of each
-// scale dword from the byte offset the dword was loaded for.  LDS reads only:
-// the scales are put in both halves by the first unpack of the stage.
-__device__ __forceinline__ void read_b(Ops& o, const TileLoads& tl, uint32_t st, int t, int wave,
-                                       int lane) {
+// Weights + scales of the stage at st; grp: scale group of the stage's first k
+// (a group of 32 kKSM k has one per half of the stage).  LDS reads only: the
+// scales are put in both halves by the first unpack of the stage.
+__device__ __forceinline__ void read_b(Ops& o, const TileLoads& tl, uint32_t st, uint32_t sc0,
+                                       int grp, int wave, int lane) {
   using L = Stage;
-  const uint32_t soff = 2 * ((kKS * t) / tl.group);
+  const int row32 = lane & 31;
+  const int g = grp + (tl.group == 32 * kKSM ? lane >> 5 : 0);
+  const uint32_t slot = sc0 + (grp / kScRun & 1) * kScSlot + ((g >> 2 & 1) * 32 + row32) * 16;
 #pragma unroll
   for (int b = 0; b < kBlk; ++b) {
 #pragma unroll
@@ -342,8 +364,8 @@ __device__ __forceinline__ void read_b(Ops& o, const TileLoads& tl, uint32_t st,
 #pragma unroll
       for (int i = 0; i < 4; ++i) o.pk[b][4 * d + i] = v[i];
     }
-    const uint32_t hsel = (tl.vs[b] + soff) & 2u;
-    o.sv[b] = lds_read<unsigned short>(st + L::kS + (wave * kBlk + b) * 256 + lane * 4 + hsel);
+    o.sv[b] = lds_read<unsigned short>(slot + (wave * kBlk + b) * 1024 + tl.vs[b] + 2 * g -
+                                       scale_src(tl, tl.vs[b], g & ~3));
   }
 }
 
@@ -380,7 +402,7 @@ __device__ __forceinline__ void sched_step() {
   }
 }
 
-// K loop of one tile over stages [tb, te) of kKS k each.  In a stage, step s's
+// K loop of one tile over te stages of kKS k each.  In a stage, step s's
 // MFMAs overlap the unpack and A-fragment reads of step s + 1.  The last step
 // is ordered by hand (scheduling fences; the compiler would otherwise hoist
 // the barrier above the MFMAs and sink the unpack below it): the wave waits
@@ -392,7 +414,7 @@ __device__ __forceinline__ void sched_step() {
 // POST MFMAs.  Every stage issues the same loads (dummies past the end), so
 // the waits take no branch; the loop ends waiting for all of them.
 template <int NRB>
-__device__ __forceinline__ void k_loop(const TileLoads& tl, int tb, int te, uint32_t lds0,
+__device__ __forceinline__ void k_loop(const TileLoads& tl, int te, uint32_t lds0,
                                        int row32, int h, int wave, int lane, const DeqRegs& dr,
                                        f32x16 (&acc)[kRBMax][kBlk]) {
   using L = Stage;
@@ -403,21 +425,25 @@ __device__ __forceinline__ void k_loop(const TileLoads& tl, int tb, int te, uint
   constexpr int COVER = PRE >= 8 ? 3 : (PRE >= 4 ? 2 : 1);  // MFMAs under the weight reads
   constexpr int VPM = PRE > COVER ? (40 + PRE - COVER - 1) / (PRE - COVER) : 40;
   Ops o;
-  issue_stage<NRB>(tl, tb, lds0, wave, true);
-  issue_stage<NRB>(tl, tb + 1 < te ? tb + 1 : tb, lds0 + L::kSize, wave, tb + 1 < te);
+  const uint32_t sc0 = lds0 + kNST * L::kSize;
+  int grp = kKS / tl.group;  // scale group of the newest stage issued
+  issue_stage<NRB>(tl, 0, 0, lds0, sc0, wave, h, true);
+  issue_stage<NRB>(tl, 1 < te ? 1 : 0, grp, lds0 + L::kSize, sc0, wave, h, 1 < te);
   wait_vmcnt<LPS>();
   stage_barrier();
-  read_b(o, tl, lds0, tb, wave, lane);
+  read_b(o, tl, lds0, sc0, 0, wave, lane);
   deq_step(o, 0, 0, dr);
   read_a<NRB>(o, 0, lds0, 0, row32, h);
   int sc = 0;  // LDS stage of stage t
-  for (int t = tb; t < te; ++t) {
+  for (int t = 0; t < te; ++t) {
     const int s1 = sc + 1 == kNST ? 0 : sc + 1;
     const int s2 = s1 + 1 == kNST ? 0 : s1 + 1;
     const uint32_t cur = lds0 + sc * L::kSize;
     const uint32_t nxt = lds0 + s1 * L::kSize;
     const bool ahead = t + 2 < te;  // uniform
-    issue_stage<NRB>(tl, ahead ? t + 2 : t, lds0 + s2 * L::kSize, wave, ahead);
+    const int grp1 = grp;           // scale group of stage t + 1
+    grp = kKS * (t + 2) / tl.group;
+    issue_stage<NRB>(tl, ahead ? t + 2 : t, grp, lds0 + s2 * L::kSize, sc0, wave, h, ahead);
 #pragma unroll
     for (int s = 0; s < kSteps - 1; ++s) {
       // step s + 1's A fragments and unpack under step s's MFMAs
@@ -428,7 +454,7 @@ __device__ __forceinline__ void k_loop(const TileLoads& tl, int tb, int te, uint
       __builtin_amdgcn_sched_barrier(0);
     }
     wait_vmcnt<LPS>();
-    read_b(o, tl, nxt, t + 1, wave, lane);
+    read_b(o, tl, nxt, sc0, grp1, wave, lane);
     __builtin_amdgcn_sched_barrier(0);
     mfma_range<0, COVER>(o, 1, acc);
     __builtin_amdgcn_sched_barrier(0);
@@ -598,7 +624,7 @@ __device__ __forceinline__ void tile_k(TileLoads& tl, int rows, long ld_x, int n
                                        f32x16 (&acc)[kRBMax][kBlk]) {
 #pragma unroll
   for (int j = 0; j < a_loads<NRB>(); ++j) tl.va[j] = a_offset<NRB>(j, wave, lane, rows, ld_x);
-  k_loop<NRB>(tl, 0, nst, lds0, row32, h, wave, lane, dr, acc);
+  k_loop<NRB>(tl, nst, lds0, row32, h, wave, lane, dr, acc);
 }
 
 // Stores row block rb of the tile's output: lane holds column n (+ 32 ob),
@@ -638,8 +664,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kOccW, kOcc
   static_assert(RBM == 4 || RBM == 8, "M-tile of 128 or 256 tokens");
   constexpr int BM = 32 * RBM;
   constexpr int WN = kWaves * 32 * kBlk / MATS;  // output columns per tile
-  using L = Stage;
-  __shared__ __align__(16) unsigned char lds[kNST * L::kSize];
+  __shared__ __align__(16) unsigned char lds[kLdsBytes];
   __shared__ int toff[kMaxProb + 1];   // full M-tiles, prefix
   __shared__ int thalf[kMaxProb + 1];  // tail M-tiles (0 / 1 per problem), prefix
   __shared__ int twt[kMaxProb];        // row blocks of each problem's tail M-tile
@@ -798,7 +823,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kOccW, kOcc
     tl.px = pr.x + (long)m0 * A.ld_x + k0;
     tl.nx = (int)(rows * A.ld_x * 2 - 2 * k0);
     tl.nq = N * A.ld_q - k0 / 2;
-    tl.ns = (N * A.ld_s - k0 / A.group) * 2;
+    tl.ns = ((N * A.ld_s - k0 / A.group) * 2 + 3) & ~3;
     tl.group = A.group;
 #pragma unroll
     for (int b = 0; b < kBlk; ++b) {
@@ -808,7 +833,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kOccW, kOcc
       tl.ps[b] = pr.s[mt] + k0 / A.group;
       const bool ok = row < N;
       tl.vq[b] = ok ? (uint32_t)(row * A.ld_q + 16 * kKSM * h) : kOOB;
-      tl.vs[b] = ok ? (uint32_t)(2 * (row * A.ld_s + (A.group == 32 * kKSM ? h : 0))) : kOOB;
+      tl.vs[b] = (uint32_t)(2 * min(row, N - 1) * A.ld_s);
     }
     f32x16 acc[kRBMax][kBlk];
 #pragma unroll
@@ -925,6 +950,7 @@ static int gemm_shape_ok(long N, long K, long group, long ld_q, long ld_s) {
   if (K <= 0 || K % kKS != 0 || group <= 0 || K % group != 0) return 0;
   if (group != 32 * kKSM && group % kKS != 0) return 0;
   if (ld_q % 16 != 0) return 0;
+  if (N <= 8) return 0;  // at least 16 bytes of scales (scale_src)
   if (N * ld_q >= (long)kOOB || N * ld_s * 2 >= (long)kOOB) return 0;
   return 1;
 }
