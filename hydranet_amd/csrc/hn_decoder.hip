@@ -31,7 +31,7 @@ constexpr int kMaxGate = 16;  // router experts the norm kernel can score
 // go out together and the E wave reductions are interleaved.
 // UNP: the residual res is the row's MoE output, computed here from the
 // down projection's four fp32 K-slice partials and the routing (the ordered
-// weighted sum of moe_unpermute_kernel<4>, unp_select / unp_cols), instead of
+// weighted sum of moe_unpermute_kernel<4>, unp_select / unp_cols_split), instead of
 // read: the MoE block's last launch and the next RMSNorm in one.
 struct UnpSrc {
   const float* part;  // [kHnDownSplit][rows][ld_y] fp32
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(
       if (UNP || rr) {
         half8_t b;
         if constexpr (UNP)
-          b = unp_cols<kHnDownSplit>(nullptr, U.part, U.ks_stride, U.ld_y, upos, uwt, un, 8 * j);
+          b = unp_cols_split<kHnDownSplit>(U.part, U.ks_stride, U.ld_y, upos, uwt, un, 8 * j);
         else
           b = rr[j];
 #pragma unroll

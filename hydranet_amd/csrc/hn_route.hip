@@ -91,6 +91,67 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const h16* __restric
 // scores: the lower group), and the row is written back with -inf for every
 // expert of the other groups (their sigmoid is then exactly 0, the
 // reference's masked score).
+// The same sums for many dot products: a wave takes LT tokens x 4 experts, so
+// a row is read once for several products.  Each sum keeps its order (per lane,
+// then pairs 32, 16, .. 1 apart; a pair's two sums are the same number), so the
+// bits are router_logits_kernel's: the first steps halve the sums each lane
+// still carries, lane l ending with sum l LT / 16.  Bound by the rows' reads
+// from L2 until the waves are too few to hide their latency: 301 tokens x 128
+// experts of 4096 (fp32) 36 us with one product per wave, 23 in tiles of 4 x
+// 4, 33 of 8 x 4; 2048 x 8 (fp16) 16.5, 16 (4 x 4), 12.4 (2 x 4).
+constexpr int kLogE = 4;
+template <typename TW, bool ROUND16, int LT>
+__global__ __launch_bounds__(256) void router_logits_tile_kernel(
+    const h16* __restrict__ h, long ld_h, const TW* __restrict__ w, long ld_w,
+    float* __restrict__ logits, int T, int E, int H) {
+  constexpr int N = LT * kLogE;
+  const int lane = threadIdx.x & 63;
+  const int ne = (E + kLogE - 1) / kLogE;
+  const long wid = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int t0 = (int)(wid / ne) * LT, e0 = (int)(wid % ne) * kLogE;
+  if (t0 >= T) return;  // whole wave
+  const h16* hr[LT];
+  const TW* wr[kLogE];
+#pragma unroll
+  for (int i = 0; i < LT; ++i) hr[i] = h + (long)(t0 + i < T ? t0 + i : T - 1) * ld_h;
+#pragma unroll
+  for (int i = 0; i < kLogE; ++i) wr[i] = w + (long)(e0 + i < E ? e0 + i : E - 1) * ld_w;
+  float acc[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) acc[i] = 0.f;
+#pragma unroll(LT == 2 ? 4 : 2)
+  for (int k = lane * 8; k < H; k += 512) {
+    float a[LT][8], b[kLogE][8];
+#pragma unroll
+    for (int i = 0; i < LT; ++i) load8f<h16>(hr[i] + k, a[i]);
+#pragma unroll
+    for (int i = 0; i < kLogE; ++i) load8f<TW>(wr[i] + k, b[i]);
+#pragma unroll
+    for (int i = 0; i < LT; ++i)
+#pragma unroll
+      for (int q = 0; q < kLogE; ++q)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          acc[i * kLogE + q] = __builtin_fmaf(a[i][j], b[q][j], acc[i * kLogE + q]);
+  }
+  int off = 32;
+#pragma unroll
+  for (int half = N / 2; half >= 1; half >>= 1, off >>= 1) {
+    const bool up = lane & off;
+#pragma unroll
+    for (int i = 0; i < half; ++i) {
+      const float keep = up ? acc[i + half] : acc[i], send = up ? acc[i] : acc[i + half];
+      acc[i] = keep + __shfl_xor(send, off, 64);
+    }
+  }
+  float v = acc[0];
+  for (; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+  const int i = lane / (64 / N), t = t0 + i / kLogE, e = e0 + i % kLogE;
+  if (lane % (64 / N) == 0 && t < T && e < E)
+    logits[(long)t * E + e] = ROUND16 ? (float)(h16)v : v;
+}
+constexpr long kLogTileMin = 16384;  // products
+
 __global__ __launch_bounds__(256) void router_group_limit_kernel(
     const float* __restrict__ logits, int T, int E, int n_group, int topk_group,
     float* __restrict__ out) {
@@ -164,16 +225,38 @@ __global__ __launch_bounds__(kPermThreads) void moe_permute_kernel(
     if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
-  if (tid == 0) {
-    int acc = 0, na = 0;
-    for (int e = 0; e < E; ++e) {
-      off[e] = acc;
-      offsets[e] = acc;
-      if (cnt[e] > 0) active[na++] = e;
-      acc += cnt[e];
+  // offsets and active experts: prefix sums over the counts by one wave, four
+  // experts per lane (one thread's walk over 128 experts took 9 of 16 us)
+  if (wave == 0) {
+    int c[kMaxExperts / 64], sum = 0, na = 0;
+#pragma unroll
+    for (int i = 0; i < kMaxExperts / 64; ++i) {
+      c[i] = cnt[lane * (kMaxExperts / 64) + i];  // 0 at E and above
+      sum += c[i];
+      na += c[i] > 0;
     }
-    offsets[E] = acc;
-    *n_active = na;
+    int acc = sum, act = na;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int s = __shfl_up(acc, d, 64), a = __shfl_up(act, d, 64);
+      if (lane >= d) acc += s, act += a;
+    }
+    if (lane == 63) {
+      offsets[E] = acc;
+      *n_active = act;
+    }
+    acc -= sum;
+    act -= na;
+#pragma unroll
+    for (int i = 0; i < kMaxExperts / 64; ++i) {
+      const int e = lane * (kMaxExperts / 64) + i;
+      if (e < E) {
+        off[e] = acc;
+        offsets[e] = acc;
+        if (c[i] > 0) active[act++] = e;
+        acc += c[i];
+      }
+    }
   }
   __syncthreads();
   for (int base = 0; base < n; base += kPermThreads) {
@@ -230,7 +313,7 @@ __global__ __launch_bounds__(256) void moe_gather_kernel(const h16* __restrict__
 
 // Workgroup (token, column block): each thread owns 8 consecutive columns
 // per pass (blockDim.x * 8 columns per block and pass, gridDim.y blocks
-// interleaved over H); the sum is unp_select / unp_cols (hn_unpermute.h).
+// interleaved over H); the sum is that of hn_unpermute.h.
 // KS = 0: y is fp16 [rows, ld_y]; KS > 0: y is given as KS fp32 partial sums
 // part[j * ks_stride + row * ld_y] (a K-split down projection), added in
 // slice order and rounded to fp16 once: the expert output the unsplit kernel
@@ -244,13 +327,21 @@ __global__ __launch_bounds__(256) void moe_unpermute_kernel(
   const int t = blockIdx.x;
   int pos[kMaxTopK];
   float wt[kMaxTopK];
-  const int n = unp_select(t, inv, idx, w, k, pos, wt);
+  int n;
+  if constexpr (KS == 0)
+    n = unp_select_wave(t, inv, idx, w, k, pos, wt);
+  else
+    n = unp_select(t, inv, idx, w, k, pos, wt);
   for (int c = (blockIdx.y * blockDim.x + threadIdx.x) * 8; c < H;
        c += gridDim.y * blockDim.x * 8) {
     // the shared expert's row is loaded with the first batch of rows
     half8_t sv = {0, 0, 0, 0, 0, 0, 0, 0};
     if (shared) sv = *reinterpret_cast<const half8_t*>(shared + (long)t * ld_sh + c);
-    half8_t acc = unp_cols<KS>(y, part, ks_stride, ld_y, pos, wt, n, c);
+    half8_t acc;
+    if constexpr (KS == 0)
+      acc = unp_cols(y, ld_y, pos, wt, n, c);
+    else
+      acc = unp_cols_split<KS>(part, ks_stride, ld_y, pos, wt, n, c);
     if (shared) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[j] = (h16)((float)sv[j] + (float)acc[j]);
@@ -501,9 +592,26 @@ extern "C" int hn_router_logits(const void* h, long ld_h, const void* w, long ld
   HN_ARG_CHECK(al16(w) && (w_dtype == 0 ? ld_w % 8 == 0 : ld_w % 4 == 0),
                "hn_router_logits: weight rows must be 16-byte aligned");
   if (T == 0) return 0;
-  const long waves = T * E;
-  dim3 grid(hn_cdiv(waves, 4)), block(256);
   hipStream_t s = (hipStream_t)stream;
+  dim3 block(256);
+  // Tiles once they alone give every SIMD a wave: below, one product per wave
+  // is spread wider.
+  if (T * E >= kLogTileMin) {
+    const int lt = w_dtype == 0 ? 2 : 4;
+    dim3 grid(hn_cdiv((long)hn_cdiv(T, lt) * hn_cdiv(E, kLogE), 4));
+    if (w_dtype == 0)
+      hipLaunchKernelGGL((router_logits_tile_kernel<h16, true, 2>), grid, block, 0, s,
+                         (const h16*)h, ld_h, (const h16*)w, ld_w, (float*)logits, (int)T, (int)E,
+                         (int)H);
+    else
+      hipLaunchKernelGGL((router_logits_tile_kernel<float, false, 4>), grid, block, 0, s,
+                         (const h16*)h, ld_h, (const float*)w, ld_w, (float*)logits, (int)T,
+                         (int)E, (int)H);
+    HN_LAUNCH_CHECK("hn_router_logits");
+    return 0;
+  }
+  const long waves = T * E;
+  dim3 grid(hn_cdiv(waves, 4));
   if (w_dtype == 0)
     hipLaunchKernelGGL((router_logits_kernel<h16, true>), grid, block, 0, s, (const h16*)h, ld_h,
                        (const h16*)w, ld_w, (float*)logits, (int)T, (int)E, (int)H);
