@@ -24,7 +24,8 @@
 //  * Activations go L2 -> LDS directly (buffer_load ... lds) into two stage
 //    slots, rows XOR-swizzled by 16-byte chunk so the A reads are free of bank
 //    conflicts; one barrier per stage.
-//  * K is split over workgroups where the tiles alone would leave CUs idle: the
+//  * Where the tiles alone would leave CUs idle, K is split over the waves of a
+//    workgroup (mid_kwave_kernel), or over workgroups where that does not apply: the
 //    splits store fp32 partials, and the last of a tile to arrive (per wave,
 //    hn_arrive) sums them in split order and writes the result, all of a
 //    thread's loads in flight; grouped launches leave them to the MoE unpermute.
@@ -195,7 +196,7 @@ template <> struct ScaleVec<2> { typedef uint32_t T; };
 template <> struct ScaleVec<8> { typedef u32x4 T; };
 
 // V scales per load; cnt scales per row from element e0 of the row.
-template <int MATS, int V>
+template <int MATS, int V, int PITCH = kScalePitch>
 __device__ __forceinline__ void stage_scales_v(const void* const (&ps)[2], int ns, int N, int ld_s,
                                                int nw, int e0, int cnt, uint32_t dst, int lane) {
   const int per_row = (cnt + V - 1) / V;
@@ -210,7 +211,7 @@ __device__ __forceinline__ void stage_scales_v(const void* const (&ps)[2], int n
     typename ScaleVec<V>::T v;
     const uint32_t off0 = second ? kOOB : off, off1 = second ? off : kOOB;
     __attribute__((address_space(3))) char* p =
-        (__attribute__((address_space(3))) char*)nullptr + dst + r * (kScalePitch * 2) + 2 * c;
+        (__attribute__((address_space(3))) char*)nullptr + dst + r * (PITCH * 2) + 2 * c;
     if constexpr (V == 8) {
       u32x4 v4 = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r0, off0, 0, 0));
       if (MATS == 2)
@@ -256,7 +257,7 @@ __device__ __forceinline__ void issue_a(const uint32_t (&va)[NRB], const TileSrc
 // One stage: NRB x kTN blocks of 16 tokens x 16 weight rows over 128 k.  Lane
 // (t = l % 16, c = l / 16) supplies A[token t][k 32 c + 8 d ..] at step d.
 // sc: LDS address of the scale of the lane's row in tile 0.
-template <int NRB, bool SC>
+template <int NRB, bool SC, int PITCH = kScalePitch>
 __device__ __forceinline__ void compute_stage(const WStage& ws, uint32_t st, uint32_t sc, int col,
                                               int q, const DeqRegs& dr,
                                               float4_t (&acc)[NRB][kTN]) {
@@ -264,7 +265,7 @@ __device__ __forceinline__ void compute_stage(const WStage& ws, uint32_t st, uin
   float4_t tmp[NRB][kTN];
   uint32_t sv[kTN];
 #pragma unroll
-  for (int b = 0; b < kTN; ++b) sv[b] = lds_read<uint16_t>(sc + b * 16 * kScalePitch * 2);
+  for (int b = 0; b < kTN; ++b) sv[b] = lds_read<uint16_t>(sc + b * 16 * PITCH * 2);
   half8_t a[2][NRB];  // step d + 1's A reads go out before step d's MFMAs
   const uint32_t row = st + col * kRowB;
 #pragma unroll
@@ -635,6 +636,183 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+// ---------------------------------------------------------------------------
+// One problem of few tiles: K split over the eight waves of a workgroup.
+//
+// A K split over workgroups costs about 8 us of its own (partials out to memory,
+// counter, read back: 64 x 6144 x 4096 takes 22.8 us in 4 splits of 8 stages and
+// 31.1 us in one of 32), and a workgroup of a short K has little in flight.  So a
+// workgroup takes a tile of 64 weight rows x 32 tokens whole and its waves a K
+// range each: every wave stages its own activations (no barrier in the K loop, two
+// slots as above) and the partials meet in LDS, summed in K order.  The
+// activations are read once per 64 weight rows instead of once per 256, from L2.
+// us before / now: 64 x 6144 x 4096 24.9 / 11.8, 64 x 4096 x 1408 19.0 / 6.9,
+// 37 x 4096 x 14336 34.1 / 29.2, 333 x 4096 x 4096 group 64 44.4 / 28.9.  Bound by
+// the stages' latency (about 1.7 us each at 14 per wave); a third register buffer of
+// weights, two stages ahead, gave nothing (32.9 against 32.7 at 128 x 4096 x 14336,
+// 12.6 against 11.9 at 64 x 6144 x 4096).
+// ---------------------------------------------------------------------------
+constexpr int kKWaves = 8;
+constexpr int kKScales = 16;                       // scales per row of a wave's K range at most
+constexpr int kKPitch = kKScales + 2;
+constexpr int kKSlots = 2 * 2 * 16 * kRowB;        // per wave: two slots of 32 tokens
+constexpr int kKScaleBytes = kTN * 16 * kKPitch * 2;
+static_assert(kKSlots >= 2 * kTN * 4 * 64 * 4, "a wave's partials fit its slots");
+
+template <int MATS, int NRB, bool SC>
+__device__ __forceinline__ void kwave_tile(const MidArgs& A, const Item& it, uint32_t lds0,
+                                           int wave, int lane, const DeqRegs& dr) {
+  constexpr uint32_t kStageB = NRB * 16 * kRowB;
+  constexpr int kLoads = 4 * NRB;  // 1 KiB activation loads of a wave and stage
+  const int col = lane & 15, q = lane >> 4;
+  const int N = A.N, s0 = it.sb, s1 = it.se;
+  const int nw = it.ntile * (kTN * 16 / MATS);
+  TileSrc t;
+  t.px = it.x;
+  t.nx = (int)(((long)(it.rows - 1) * A.ld_x + A.K) * 2);
+  t.nq = N * A.ld_q;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) t.pq[m] = it.q[MATS == 2 ? m : 0];
+#pragma unroll
+  for (int b = 0; b < kTN; ++b) {
+    const int row = nw + 16 * (MATS == 2 ? b % (kTN / 2) : b) + col;
+    t.vq[b] = row < N ? (uint32_t)(row * A.ld_q + 16 * q) : kOOB;
+  }
+  // wave-private rows: the layout of a_offsets with one wave's loads covering all
+  uint32_t va[kLoads];
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) {
+    const int L = j * 64 + lane, r = L >> 4, c = (L & 15) ^ (r & 15);
+    va[j] = (uint32_t)(min(r, it.rows - 1) * (int)A.ld_x * 2 + 16 * c);
+  }
+  const uint32_t st0 = lds0 + wave * kKSlots;
+  auto issue_rows = [&](int s, uint32_t st, bool real) {
+    const __amdgpu_buffer_rsrc_t r = rsrc(t.px, real ? t.nx : 0);
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) dma_b128(r, va[j], kRowB * s, st + j * 1024);
+  };
+  float4_t acc[NRB][kTN];
+#pragma unroll
+  for (int rb = 0; rb < NRB; ++rb)
+#pragma unroll
+    for (int b = 0; b < kTN; ++b) acc[rb][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+  WStage ws0, ws1;
+  issue_rows(s0, st0, true);
+  __builtin_amdgcn_sched_barrier(0);
+  issue_w<MATS>(ws0, t, s0, true);
+  __builtin_amdgcn_sched_barrier(0);
+  const int sps = kStageK / A.group;
+  const uint32_t scw = lds0 + (uint32_t)(kKWaves * kKSlots) + wave * kKScaleBytes;
+  {
+    const void* const ps[2] = {it.s[0], it.s[MATS - 1]};
+    const int ns = N * A.ld_s * 2, cnt = (s1 - s0) * sps, e0 = s0 * sps;
+    if (A.sv == 8)  // uniform
+      stage_scales_v<MATS, 8, kKPitch>(ps, ns, N, A.ld_s, nw, e0, cnt, scw, lane);
+    else if (A.sv == 2)
+      stage_scales_v<MATS, 2, kKPitch>(ps, ns, N, A.ld_s, nw, e0, cnt, scw, lane);
+    else
+      stage_scales_v<MATS, 1, kKPitch>(ps, ns, N, A.ld_s, nw, e0, cnt, scw, lane);
+  }
+  uint32_t sc = scw + col * (kKPitch * 2) + 2 * (q * sps / 4);
+  // as k_loop's stage, the slots being the wave's own: its loads landed and its
+  // LDS reads returned are all that a slot's reuse needs
+  auto stage = [&](int s, const WStage& cur, WStage& nxt, uint32_t stc, uint32_t stn) {
+    wait_vmcnt<kWLoads>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const bool more = s + 1 < s1;  // uniform
+    issue_rows(s + 1, stn, more);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_w<MATS>(nxt, t, s + 1, more);
+    __builtin_amdgcn_sched_barrier(0);
+    compute_stage<NRB, SC, kKPitch>(cur, stc, sc, col, q, dr, acc);
+    sc += 2 * sps;
+  };
+  int s = s0;
+  for (; s + 2 <= s1; s += 2) {
+    stage(s, ws0, ws1, st0, st0 + kStageB);
+    stage(s + 1, ws1, ws0, st0 + kStageB, st0);
+  }
+  if (s < s1) {
+    wait_vmcnt<kWLoads>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    compute_stage<NRB, SC, kKPitch>(ws0, st0, sc, col, q, dr, acc);
+  }
+  wait_vmcnt<0>();  // requests past the end have landed: the slots are free
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+
+  // partials by (register, lane) into the wave's slots; wave w sums register r =
+  // w % 4 of two tiles (a gate and up pair with MATS 2)
+  auto cell = [&](int w, int rb, int b, int r) {
+    return (__attribute__((address_space(3))) float*)(
+        (__attribute__((address_space(3))) char*)nullptr + lds0 + w * kKSlots +
+        (((rb * kTN + b) * 4 + r) * 64 + lane) * 4);
+  };
+#pragma unroll
+  for (int rb = 0; rb < NRB; ++rb)
+#pragma unroll
+    for (int b = 0; b < kTN; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) *cell(wave, rb, b, r) = acc[rb][b][r];
+  __syncthreads();
+  const int r = wave & 3, h = wave >> 2;
+#pragma unroll
+  for (int rb = 0; rb < NRB; ++rb) {
+    float v[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int b = MATS == 2 ? h + u * (kTN / 2) : 2 * h + u;
+      v[u] = 0.f;
+#pragma unroll
+      for (int w = 0; w < kKWaves; ++w) v[u] += *cell(w, rb, b, r);
+    }
+    const int m = 16 * rb + 4 * q + r;
+    if (m < it.rows) {
+#pragma unroll
+      for (int u = 0; u < 2 / MATS; ++u) {
+        const int n = nw + 16 * (MATS == 2 ? h : 2 * h + u) + col;
+        if (n < N)
+          it.out[(long)m * A.ld_o + n] = MATS == 2 ? swiglu16(v[0], v[1]) : (h16)v[u];
+      }
+    }
+  }
+}
+
+// One tile per workgroup: n-tile bid / mtiles, m-tiles fastest on one XCD.
+template <int MATS, bool SC>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void mid_kwave_kernel(
+    MidArgs A) {
+  __shared__ __align__(16) unsigned char lds[kKWaves * (kKSlots + kKScaleBytes)];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t*)lds;
+  DeqRegs dr;
+  dr.m_pair = A.m_pair;
+  dr.magic = hn_vgpr(A.magic);
+  dr.mul = hn_vgpr(0x2C003C00u);  // half2(1, 0.0625)
+  dr.add = hn_vgpr(0xD480E408u);  // half2(-1032, -72)
+  const int nwg = gridDim.x, bid = blockIdx.x;
+  const int vid = (nwg % 8 == 0) ? (bid % 8) * (nwg / 8) + bid / 8 : bid;
+  const int nmt = (A.M + 31) >> 5;
+  Item it;
+  it.ntile = vid / nmt;
+  const int mtile = vid - it.ntile * nmt;
+  const int T = A.K / kStageK;
+  it.sb = T * wave / kKWaves;
+  it.se = T * (wave + 1) / kKWaves;
+  it.q[0] = A.q[0]; it.s[0] = A.s[0];
+  it.q[1] = A.q[1]; it.s[1] = A.s[1];
+  // rows dealt evenly to the m-tiles in blocks of 16
+  const int blocks = (A.M + 15) >> 4;
+  const int b0 = blocks * mtile / nmt, b1 = blocks * (mtile + 1) / nmt;
+  it.nrb = b1 - b0;
+  it.rows = min(16 * it.nrb, A.M - 16 * b0);
+  it.x = A.x + (long)(16 * b0) * A.ld_x;
+  it.out = A.out + (long)(16 * b0) * A.ld_o;
+  if (it.nrb == 1) kwave_tile<MATS, 1, SC>(A, it, lds0, wave, lane, dr);
+  else kwave_tile<MATS, 2, SC>(A, it, lds0, wave, lane, dr);
+}
+
 // out[m, n] = the ks partials of (m, n) summed in split order; four columns per
 // thread, all of its loads in flight.
 __global__ __launch_bounds__(256) void mid_reduce_kernel(const float* __restrict__ part,
@@ -669,7 +847,7 @@ namespace {
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// Resident workgroups the splits aim at: two per CU.
+// Resident workgroups of mid_kernel: two per CU.
 int slots() { return 2 * hn_device_cus(); }
 
 // Single problems.  Work in units of one tile's stage.  Measured on MI355X
@@ -690,7 +868,31 @@ struct MidPlan {
   bool ok;
   int rbm;  // 16-token blocks per tile
   int ks;   // K splits
+  bool kw;  // K over the waves of a workgroup (mid_kwave_kernel)
 };
+
+long kwave_tiles(int mats, long M, long N) {
+  return (M + 31) / 32 * ((N * mats + kTN * 16 - 1) / (kTN * 16));
+}
+
+// Where mid_kwave_kernel takes a problem: a stage for every wave, the scales of a
+// wave's range in LDS, and a few rounds of workgroups (one per CU), past which its
+// 32-token tiles unpack the weights too often.  us against the kernels below (tiles;
+// M x N x K):
+//   one matrix, 8 - 15 stages, 2 rounds:  448 (200 x 4096 x 1408)    12 /  18
+//                                         832 (400 x 4096 x 1408)    21 /  18
+//   to 64 stages, 5 rounds:              1056 (333 x 6144 x 4096)    44 /  55
+//                                        1280 (640 x 4096 x 4096)    53 /  58
+//                                        1568 (200 x 14336 x 4096)   66 /  61
+//   more, 3 rounds:                       704 (333 x 4096 x 14336)   85 /  89
+//   gate and up, 2 rounds (the whole expert): 448 (17 x 14336 x 4096)  58 / 66,
+//     704 (500 x 1408 x 4096) 49 / 49, 896 (37 x 14336 x 4096) 73 / 66,
+//     968 (700 x 1408 x 4096) 67 / 55.
+bool kwave_ok(int mats, long M, long N, long T, long sps) {
+  const long rounds = mats == 2 || T < 2 * kKWaves ? 2 : T <= 64 ? 5 : 3;
+  return T >= kKWaves && (T + kKWaves - 1) / kKWaves * sps <= kKScales &&
+         kwave_tiles(mats, M, N) <= rounds * hn_device_cus();
+}
 
 MidPlan mid_plan(int mats, long M, long N, long K, long group) {
   MidPlan p{};
@@ -698,15 +900,23 @@ MidPlan mid_plan(int mats, long M, long N, long K, long group) {
     return p;
   const long T = K / kStageK, sps = kStageK / group;
   const long nt = (N * mats + kBN - 1) / kBN;
+  if (kwave_ok(mats, M, N, T, sps)) {
+    p.kw = p.ok = true;
+    p.rbm = 2;
+    p.ks = 1;
+    return p;
+  }
   const long t32 = (M + 31) / 32 * nt, t64 = (M + 63) / 64 * nt;
   const bool small = t32 * T <= kUnits32 || t32 == t64;
   if (!small && (t64 > slots() || t64 * T > kUnits64)) return p;
   p.rbm = small ? 2 : 4;
   const long tiles = small ? t32 : t64;
-  // K splits fill one round of workgroups with at least two stages each; an even
-  // split (whole scale vectors per load) where one comes within half of that
+  // K splits to one workgroup per CU (at two per CU the splits' reduction costs more
+  // than they give: the expert of 4096 x 14336 at 37 rows 74.0 us, 66.0 with gate/up
+  // whole; 37 x 4096 x 14336 group 32 40.7 / 37.1), of at least two stages each; an
+  // even split (whole scale vectors per load) where one comes within half of that
   const long kmin = (T * sps + kMaxScales - 1) / kMaxScales;
-  long lim = slots() / tiles;
+  long lim = hn_device_cus() / tiles;
   if (lim > T / 2) lim = T / 2;
   if (N % 4 != 0) lim = 1;  // the reduction reads four columns at a time
   if (lim < 1) lim = 1;
@@ -805,10 +1015,23 @@ extern "C" int hn_mid_linear_impl(int mats, const void* x, long ld_x, const void
   A.q[1] = (const uint8_t*)q1; A.s[1] = (const h16*)s1;
   A.out = (h16*)out;
   A.ld_o = ld_o;
-  fill_common(A, N, K, group, ld_q, ld_s, p.ks, scale_vec(K, ld_s, group, p.ks, s0, s1));
+  fill_common(A, N, K, group, ld_q, ld_s, p.ks,
+              scale_vec(K, ld_s, group, p.kw ? kKWaves : p.ks, s0, s1));
   A.part = work ? (float*)((char*)work + kPartOffset) : nullptr;
   A.part_rows = M;
   hipStream_t s = (hipStream_t)stream;
+  if (p.kw) {
+    const dim3 grid((unsigned)kwave_tiles(mats, M, N)), block(64 * kKWaves);
+    if (mats == 2) {
+      if (group == kStageK) hipLaunchKernelGGL((mid_kwave_kernel<2, true>), grid, block, 0, s, A);
+      else hipLaunchKernelGGL((mid_kwave_kernel<2, false>), grid, block, 0, s, A);
+    } else {
+      if (group == kStageK) hipLaunchKernelGGL((mid_kwave_kernel<1, true>), grid, block, 0, s, A);
+      else hipLaunchKernelGGL((mid_kwave_kernel<1, false>), grid, block, 0, s, A);
+    }
+    HN_LAUNCH_CHECK("hn_mid_linear");
+    return 0;
+  }
   const long tm = 16 * p.rbm;
   const long tiles = (M + tm - 1) / tm * ((N * mats + kBN - 1) / kBN);
   const long items = tiles * p.ks;
