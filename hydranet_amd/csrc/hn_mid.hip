@@ -882,15 +882,19 @@ long kwave_tiles(int mats, long M, long N) {
 //   one matrix, 8 - 15 stages, 2 rounds:  448 (200 x 4096 x 1408)    12 /  18
 //                                         832 (400 x 4096 x 1408)    21 /  18
 //   to 64 stages, 5 rounds:              1056 (333 x 6144 x 4096)    44 /  55
-//                                        1280 (640 x 4096 x 4096)    53 /  58
 //                                        1568 (200 x 14336 x 4096)   66 /  61
 //   more, 3 rounds:                       704 (333 x 4096 x 14336)   85 /  89
 //   gate and up, 2 rounds (the whole expert): 448 (17 x 14336 x 4096)  58 / 66,
 //     704 (500 x 1408 x 4096) 49 / 49, 896 (37 x 14336 x 4096) 73 / 66,
 //     968 (700 x 1408 x 4096) 67 / 55.
+// Above kKRows rows the gain is small (640 x 4096 x 4096 53 / 58, 1000 x 1408 x 4096
+// 36 / 42) and the reductions across workgroups, which need a workspace and its
+// counters anyway, stay the only path.
+constexpr long kKRows = 480;
+
 bool kwave_ok(int mats, long M, long N, long T, long sps) {
   const long rounds = mats == 2 || T < 2 * kKWaves ? 2 : T <= 64 ? 5 : 3;
-  return T >= kKWaves && (T + kKWaves - 1) / kKWaves * sps <= kKScales &&
+  return M <= kKRows && T >= kKWaves && (T + kKWaves - 1) / kKWaves * sps <= kKScales &&
          kwave_tiles(mats, M, N) <= rounds * hn_device_cus();
 }
 

@@ -44,9 +44,9 @@ def _close(y, ref):
     (65, 100, 1408, 128), (40, 1408, 1408, 128), (200, 4096, 14336, 128), (333, 4096, 4096, 64),
     (48, 1030, 640, 64), (19, 512, 4096, 32), (512, 1000, 2048, 32), (24, 4094, 4096, 128),
     # K over a workgroup's waves: one stage each, uneven ranges, one row past a tile,
-    # two and eight scales a load, several rounds of tiles, the most (1280) and more
+    # two and eight scales a load, several rounds of tiles, the most rows (480) and more
     (17, 70, 1024, 128), (45, 4096, 1408, 128), (33, 1030, 2176, 128), (49, 100, 2176, 64),
-    (37, 4096, 14336, 128), (127, 4096, 2048, 64), (640, 4096, 2048, 128), (641, 4096, 2048, 128),
+    (37, 4096, 14336, 128), (127, 4096, 2048, 64), (480, 4096, 2048, 128), (481, 4096, 2048, 128),
     # K over workgroups: few stages, scales past a wave's share
     (20, 256, 768, 128), (37, 512, 14336, 64), (150, 1028, 14336, 32),
 ])
