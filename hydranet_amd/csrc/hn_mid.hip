@@ -64,7 +64,7 @@ struct MidArgs {
   int N, K, group;
   int ld_q;           // packed row stride (bytes)
   int ld_s;           // scale row stride (elements)
-  int ks;             // K splits per tile; a split holds at most kMaxScales scales per row
+  int ks;             // K splits per tile
   int sv;             // scales per load when staging them (8, 2 or 1, by alignment)
   float* part;        // PART: [ks][MATS][part_rows][N] fp32
   long part_rows;
@@ -179,13 +179,16 @@ __device__ __forceinline__ void issue_w(WStage& ws, const TileSrc& t, int g, boo
 }
 constexpr int kWLoads = kTN;  // per wave and stage
 
-// The scales of the wave's 64 weight rows over its K split, copied to LDS once
-// per tile ([row][kScalePitch] fp16, the wave's own region): read per stage
-// from memory they are one 2-byte gather over 16 rows per tile and stage, which
-// costs the CU's L1 about 65 clocks against 35 for a 1 KiB weight load
-// (measured, L2-resident; the grouped gate/up of 8 experts x 25 rows 183 ->
-// 145 us without them).  A row holds at most kMaxScales of a split; the pitch
-// spreads 16 rows over the banks.
+// The scales of the wave's 64 weight rows, copied to LDS in runs of kMaxScales per
+// row ([row][kScalePitch] fp16, the wave's own region): read per stage from memory
+// they are one 2-byte gather over 16 rows per tile and stage, which costs the
+// CU's L1 about 65 clocks against 35 for a 1 KiB weight load (measured, L2-resident;
+// the grouped gate/up of 8 experts x 25 rows 183 -> 145 us without them).  A run is
+// loaded when the stages of the one before are done, which waits for the loads of
+// one stage; with K split so that one run covers a split instead (2 splits at group 64
+// and 4 at group 32 of K = 4096, whatever the tiles), the partials cost more: us
+// by splits / by runs, 1500 x 4096 x 4096 group 64 117 / 71, group 32 128 / 73;
+// 512 x 14336 x 4096 group 32 171 / 77.  The pitch spreads 16 rows over the banks.
 constexpr int kMaxScales = 32;
 constexpr int kScalePitch = kMaxScales + 2;
 constexpr int kScaleBytes = kTN * 16 * kScalePitch * 2;  // per wave
@@ -330,20 +333,25 @@ __device__ __forceinline__ void k_loop(const MidArgs& A, const Item& it, const T
   __builtin_amdgcn_sched_barrier(0);
   issue_w<MATS>(ws0, t, s0, true);
   __builtin_amdgcn_sched_barrier(0);
-  // the scales of this split (sps per stage and row), behind the first stage's loads
-  const int sps = kStageK / A.group;
+  // Scales, sps per stage and row, a run of kMaxScales per row at a time, the first
+  // behind the first stage's loads.
+  const int sps = kStageK / A.group, run = kMaxScales / sps;  // stages per run: even
   const uint32_t scw = lds0 + (uint32_t)(2 * RBM * 16 * kRowB) + wave * kScaleBytes;
-  {
+  const uint32_t sc0 = scw + col * (kScalePitch * 2) + 2 * (q * sps / 4);
+  uint32_t sc = sc0;
+  int nrun = s0;  // first stage of the run to load next
+  auto load_run = [&](int s) {
     const void* const ps[2] = {it.s[0], it.s[MATS - 1]};
-    const int ns = A.N * A.ld_s * 2, cnt = (s1 - s0) * sps, e0 = s0 * sps;
+    const int ns = A.N * A.ld_s * 2, cnt = min(s1 - s, run) * sps, e0 = s * sps;
     if (A.sv == 8)  // uniform
       stage_scales_v<MATS, 8>(ps, ns, A.N, A.ld_s, nw, e0, cnt, scw, lane);
     else if (A.sv == 2)
       stage_scales_v<MATS, 2>(ps, ns, A.N, A.ld_s, nw, e0, cnt, scw, lane);
     else
       stage_scales_v<MATS, 1>(ps, ns, A.N, A.ld_s, nw, e0, cnt, scw, lane);
-  }
-  uint32_t sc = scw + col * (kScalePitch * 2) + 2 * (q * sps / 4);
+    sc = sc0;
+    nrun = s + run;
+  };
   auto stage = [&](int s, const WStage& cur, WStage& nxt, uint32_t stc, uint32_t stn) {
     wait_vmcnt<kWLoads>();
     stage_barrier();
@@ -357,10 +365,12 @@ __device__ __forceinline__ void k_loop(const MidArgs& A, const Item& it, const T
   };
   int s = s0;
   for (; s + 2 <= s1; s += 2) {
+    if (s == nrun) load_run(s);
     stage(s, ws0, ws1, lds0, lds0 + kStageB);
     stage(s + 1, ws1, ws0, lds0 + kStageB, lds0);
   }
   if (s < s1) {  // the last of an odd number: nothing left to request
+    if (s == nrun) load_run(s);
     wait_vmcnt<kWLoads>();
     stage_barrier();
     compute_stage<NRB, SC>(ws0, lds0, sc, col, q, dr, acc);
@@ -864,6 +874,8 @@ int slots() { return 2 * hn_device_cus(); }
 // padding and idle CUs.
 constexpr long kUnits32 = 8192, kUnits64 = 16384;
 
+constexpr long kSplitStages = 32;
+
 struct MidPlan {
   bool ok;
   int rbm;  // 16-token blocks per tile
@@ -919,17 +931,25 @@ MidPlan mid_plan(int mats, long M, long N, long K, long group) {
   // than they give: the expert of 4096 x 14336 at 37 rows 74.0 us, 66.0 with gate/up
   // whole; 37 x 4096 x 14336 group 32 40.7 / 37.1), of at least two stages each; an
   // even split (whole scale vectors per load) where one comes within half of that
-  const long kmin = (T * sps + kMaxScales - 1) / kMaxScales;
   long lim = hn_device_cus() / tiles;
   if (lim > T / 2) lim = T / 2;
-  if (N % 4 != 0) lim = 1;  // the reduction reads four columns at a time
+  if (N % 4 != 0) {  // the reduction reads four columns at a time
+    if (T > kSplitStages) return p;
+    lim = 1;
+  }
   if (lim < 1) lim = 1;
   long ks = lim;
   for (long d = lim; d >= 1 && 2 * d >= lim; --d)
     if (T % d == 0) { ks = d; break; }
-  if (ks < kmin) ks = kmin;
-  while (ks < T && (T + ks - 1) / ks * sps > kMaxScales) ++ks;
-  if ((T + ks - 1) / ks * sps > kMaxScales || (ks > 1 && N % 4 != 0)) return p;
+  // past K = 8192, splits of at most 32 stages however many tiles there are (us, one
+  // split for each CU and splits of 32: 1500 x 1024 x 14336 96 / 87; gate and up
+  // of 160 x 4096 x 14336 90 / 86)
+  if (T > 2 * kSplitStages) {
+    const long m = (T + kSplitStages - 1) / kSplitStages;
+    long d = m;
+    while (d < 2 * m && T % d != 0) ++d;
+    if (ks < d) ks = T % d == 0 ? d : m;
+  }
   p.ks = (int)ks;
   p.ok = true;
   return p;

@@ -59,9 +59,31 @@ def test_linear(m, n, k, group):
     assert torch.equal(y, g.int4_linear(x, p, s, group))  # sums in split order: repeatable
 
 
+@pytest.mark.parametrize("m,n,k,group", [
+    # several runs of scales per tile: whole K and K splits, 32- and 64-token tiles, an odd
+    # number of stages with a short last run, rows of scales that start on any half word
+    (520, 2048, 4096, 32), (1030, 2048, 4096, 64), (600, 4096, 4096, 64), (700, 4096, 1408, 32),
+    (1100, 1030, 2176, 32), (300, 512, 14336, 32), (100, 512, 11008, 64), (530, 2300, 5120, 128),
+    (90, 1000, 17664, 128),
+])
+def test_linear_scale_runs(m, n, k, group):
+    print(f"[mid] scale runs m={m} n={n} k={k} group={group}", flush=True)
+    p, s = _weight(n, k, group, m + n)
+    # every group its own size, so that a scale from another group shows
+    s *= (2.0 ** (torch.arange(k // group, device="cuda") * 5 % 7 - 3)).half()
+    x = _x(m, k, m)
+    y = g.int4_linear(x, p, s, group)
+    ref, size = x.double() @ _deq(p, s).t(), x.double().abs() @ _deq(p, s).abs().t()
+    # fp32 sums of k products, below group 128 of weights rounded to fp16 (2^-11 each, all one
+    # way at worst), one fp16 rounding of the result
+    bound = (k * 2.0 ** -23 + (2.0 ** -11 if group < 128 else 0.0)) * size + 2.0 ** -10 * ref.abs() + 1e-6
+    assert bool(((y.double() - ref).abs() <= bound).all()), ((y.double() - ref).abs() / bound).max().item()
+
+
 @pytest.mark.parametrize("t,h,i,group", [(17, 512, 768, 128), (37, 4096, 14336, 128),
                                          (64, 1024, 1408, 64), (130, 640, 2048, 128),
-                                         (33, 2048, 1408, 128), (47, 2304, 1088, 64)])
+                                         (33, 2048, 1408, 128), (47, 2304, 1088, 64),
+                                         (1100, 4096, 512, 32)])
 def test_expert(t, h, i, group):
     print(f"[mid] expert t={t} h={h} i={i} group={group}", flush=True)
     ws = [_weight(a, b, group, 7 + j) for j, (a, b) in enumerate(((i, h), (i, h), (h, i)))]
