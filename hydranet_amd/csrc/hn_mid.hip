@@ -876,6 +876,24 @@ constexpr long kUnits32 = 8192, kUnits64 = 16384;
 
 constexpr long kSplitStages = 32;
 
+// Where the kernels beside these are faster (us here, theirs; M x N x K, group 128
+// unless said):
+//  * a short K, under kShort stages: K is not split (64 x 4096 x 512 in 2 splits 17.7,
+//    whole 8.3), up to 32 rows the decode kernels win (17 x 4096 x 512 7.6, 5.7; 32 x
+//    4096 x 768 12.4, 12.6; 33: 9.8, 13.4), up to 64 below half of that (64 x 8192 x
+//    256 6.6, 6.1); past 64 the GEMM where there are two tiles and more for a resident
+//    workgroup (4096 x 4096 x 512 37, 34; 512 x 14336 x 512 gate and up 43, 32; 2048 x
+//    4096 x 512 23, 35), or one up to its 128-token tile (65 x 65536 x 512 19.2, 18.5);
+//  * up to kFewRows rows the decode kernels hold a long K's activations in few K
+//    chunks: one matrix of K > 4096 over the waves, tiles for less than half of the
+//    CUs (17 x 1024 x 7680 18.7, 15.8; 20 x 4096 x 14336 32.2, 28.7), apart from even
+//    ranges of 5 to 8 stages over 64 tiles (17 x 4096 x 8192 16.4, 18.8);
+//  * up to 32 rows a product too small for the reduction across workgroups (K beyond
+//    what the waves' ranges take; mats * N * K against kFewWork): 20 x 5120 x 13824
+//    group 64 32.5, 30.3; 21 x 14336 x 7680 group 32 43.5, 43.5; 24 x 4096 x 8192 group
+//    32 24.7, 21.8; 24 x 4096 x 10240 group 64 27.0, 27.8.
+constexpr long kShort = 8, kFewRows = 21, kFewWork = 100'000'000;
+
 struct MidPlan {
   bool ok;
   int rbm;  // 16-token blocks per tile
@@ -915,8 +933,11 @@ MidPlan mid_plan(int mats, long M, long N, long K, long group) {
   if (M < 1 || N < 1 || K % kStageK != 0 || group < 32 || (group & (group - 1)) || group > kStageK)
     return p;
   const long T = K / kStageK, sps = kStageK / group;
-  const long nt = (N * mats + kBN - 1) / kBN;
+  if (T < kShort && (M <= 32 || (M <= 64 && T < kShort / 2))) return p;
+  const long nt = (N * mats + kBN - 1) / kBN, tk = kwave_tiles(mats, M, N);
   if (kwave_ok(mats, M, N, T, sps)) {
+    if (mats == 1 && M <= kFewRows && T > 32 && tk < 128 && (tk < 64 || T > 64 || T % kKWaves != 0))
+      return p;
     p.kw = p.ok = true;
     p.rbm = 2;
     p.ks = 1;
@@ -925,6 +946,7 @@ MidPlan mid_plan(int mats, long M, long N, long K, long group) {
   const long t32 = (M + 31) / 32 * nt, t64 = (M + 63) / 64 * nt;
   const bool small = t32 * T <= kUnits32 || t32 == t64;
   if (!small && (t64 > slots() || t64 * T > kUnits64)) return p;
+  if (T < kShort && M > 64 && t32 > (M <= 128 ? 1 : 2) * slots()) return p;
   p.rbm = small ? 2 : 4;
   const long tiles = small ? t32 : t64;
   // K splits to one workgroup per CU (at two per CU the splits' reduction costs more
@@ -937,7 +959,7 @@ MidPlan mid_plan(int mats, long M, long N, long K, long group) {
     if (T > kSplitStages) return p;
     lim = 1;
   }
-  if (lim < 1) lim = 1;
+  if (lim < 1 || T < kShort) lim = 1;
   long ks = lim;
   for (long d = lim; d >= 1 && 2 * d >= lim; --d)
     if (T % d == 0) { ks = d; break; }
@@ -950,6 +972,7 @@ MidPlan mid_plan(int mats, long M, long N, long K, long group) {
     while (d < 2 * m && T % d != 0) ++d;
     if (ks < d) ks = T % d == 0 ? d : m;
   }
+  if (M <= 32 && ks > 1 && mats * N * K < (M <= kFewRows ? kFewWork : kFewWork * 2 / 5)) return p;
   p.ks = (int)ks;
   p.ok = true;
   return p;
@@ -1003,6 +1026,13 @@ void launch_single(const MidArgs& A, const MidPlan& p, int grid, hipStream_t s) 
 constexpr long kRows32 = 20;
 
 }  // namespace
+
+// How a single problem is run here: 0 not at all, -1 K over the waves of a workgroup,
+// else the number of K splits over workgroups (1: whole).
+extern "C" int hn_mid_linear_plan(int mats, long M, long N, long K, long group) {
+  const MidPlan p = mid_plan(mats, M, N, K, group);
+  return !p.ok ? 0 : p.kw ? -1 : p.ks;
+}
 
 // Workspace bytes (after kPartOffset) a single problem's K splits need; 0 when
 // not handled or not split.

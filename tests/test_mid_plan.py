@@ -13,6 +13,13 @@ def _part_bytes(mats, m, n, k):
     return f(mats, m, n, k)
 
 
+def _plan(mats, m, n, k, group):
+    """0: not a product for these kernels; -1: K over a workgroup's waves; else K splits."""
+    f = _lib.lib().hn_mid_linear_plan
+    f.restype, f.argtypes = ctypes.c_int, [ctypes.c_int] + [ctypes.c_long] * 4
+    return f(mats, m, n, k, group)
+
+
 @pytest.mark.parametrize("mats,m,n,k", [(1, 1500, 4096, 4096), (1, 1024, 6144, 4096),
                                         (1, 512, 14336, 4096), (1, 2048, 4096, 1408),
                                         (2, 700, 4096, 4096), (2, 200, 14336, 4096),
@@ -22,3 +29,28 @@ def test_no_split_where_the_tiles_fill_the_chip(mats, m, n, k):
     the CUs or more."""
     assert -(-m // 64) * -(-n * mats // 256) > 128
     assert _part_bytes(mats, m, n, k) == 0
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("mats,m,n,k,want", [
+    # few stages: never split, few rows and many tiles left to the other kernels
+    (1, 17, 4096, 512, 0), (1, 32, 4096, 768, 0), (2, 17, 14336, 512, 0), (1, 64, 8192, 256, 0),
+    (1, 33, 4096, 512, 1), (2, 64, 4096, 768, 1), (1, 200, 4096, 512, 1), (1, 65, 256, 512, 1),
+    (1, 4096, 4096, 512, 0), (2, 512, 14336, 512, 0), (1, 65, 65536, 512, 0),
+    (1, 512, 14336, 512, 1),
+    # up to 21 rows of a long K in few tiles, and the rows past them
+    (1, 17, 1024, 8192, 0), (1, 21, 4096, 14336, 0), (1, 20, 5120, 13824, 0), (1, 17, 4096, 5632, 0),
+    (1, 17, 4096, 4096, -1), (1, 21, 14336, 4096, -1),
+])
+def test_left_to_the_other_kernels(mats, m, n, k, group, want):
+    assert _plan(mats, m, n, k, group) == want
+
+
+@pytest.mark.parametrize("mats,m,n,k,group,want", [
+    (1, 22, 4096, 14336, 128, -1), (1, 17, 4096, 8192, 128, -1), (1, 17, 4096, 8192, 64, -1),
+    # K beyond the waves' ranges: split over workgroups only where there is work for it
+    (1, 24, 4096, 8192, 32, 0), (1, 32, 1024, 14336, 64, 0), (2, 24, 1024, 8192, 32, 0),
+    (1, 22, 4096, 14336, 64, 16), (1, 33, 4096, 8192, 32, 8), (1, 17, 8192, 28672, 128, 8),
+])
+def test_few_rows_split_with_work_enough(mats, m, n, k, group, want):
+    assert _plan(mats, m, n, k, group) == want
