@@ -333,25 +333,9 @@ __device__ __forceinline__ void k_loop(const MidArgs& A, const Item& it, const T
   __builtin_amdgcn_sched_barrier(0);
   issue_w<MATS>(ws0, t, s0, true);
   __builtin_amdgcn_sched_barrier(0);
-  // Scales, sps per stage and row, a run of kMaxScales per row at a time, the first
-  // behind the first stage's loads.
-  const int sps = kStageK / A.group, run = kMaxScales / sps;  // stages per run: even
+  const int sps = kStageK / A.group, run = kMaxScales / sps;  // scales, stages per run: even
   const uint32_t scw = lds0 + (uint32_t)(2 * RBM * 16 * kRowB) + wave * kScaleBytes;
-  const uint32_t sc0 = scw + col * (kScalePitch * 2) + 2 * (q * sps / 4);
-  uint32_t sc = sc0;
-  int nrun = s0;  // first stage of the run to load next
-  auto load_run = [&](int s) {
-    const void* const ps[2] = {it.s[0], it.s[MATS - 1]};
-    const int ns = A.N * A.ld_s * 2, cnt = min(s1 - s, run) * sps, e0 = s * sps;
-    if (A.sv == 8)  // uniform
-      stage_scales_v<MATS, 8>(ps, ns, A.N, A.ld_s, nw, e0, cnt, scw, lane);
-    else if (A.sv == 2)
-      stage_scales_v<MATS, 2>(ps, ns, A.N, A.ld_s, nw, e0, cnt, scw, lane);
-    else
-      stage_scales_v<MATS, 1>(ps, ns, A.N, A.ld_s, nw, e0, cnt, scw, lane);
-    sc = sc0;
-    nrun = s + run;
-  };
+  uint32_t sc = 0;
   auto stage = [&](int s, const WStage& cur, WStage& nxt, uint32_t stc, uint32_t stn) {
     wait_vmcnt<kWLoads>();
     stage_barrier();
@@ -364,13 +348,24 @@ __device__ __forceinline__ void k_loop(const MidArgs& A, const Item& it, const T
     sc += 2 * sps;
   };
   int s = s0;
-  for (; s + 2 <= s1; s += 2) {
-    if (s == nrun) load_run(s);
-    stage(s, ws0, ws1, lds0, lds0 + kStageB);
-    stage(s + 1, ws1, ws0, lds0 + kStageB, lds0);
+  for (int r0 = s0; r0 < s1; r0 += run) {
+    // the run's scales, the first behind the first stage's loads
+    const int r1 = min(r0 + run, s1);
+    const void* const ps[2] = {it.s[0], it.s[MATS - 1]};
+    const int ns = A.N * A.ld_s * 2, cnt = (r1 - r0) * sps, e0 = r0 * sps;
+    if (A.sv == 8)  // uniform
+      stage_scales_v<MATS, 8>(ps, ns, A.N, A.ld_s, nw, e0, cnt, scw, lane);
+    else if (A.sv == 2)
+      stage_scales_v<MATS, 2>(ps, ns, A.N, A.ld_s, nw, e0, cnt, scw, lane);
+    else
+      stage_scales_v<MATS, 1>(ps, ns, A.N, A.ld_s, nw, e0, cnt, scw, lane);
+    sc = scw + col * (kScalePitch * 2) + 2 * (q * sps / 4);
+    for (; s + 2 <= r1; s += 2) {
+      stage(s, ws0, ws1, lds0, lds0 + kStageB);
+      stage(s + 1, ws1, ws0, lds0 + kStageB, lds0);
+    }
   }
   if (s < s1) {  // the last of an odd number: nothing left to request
-    if (s == nrun) load_run(s);
     wait_vmcnt<kWLoads>();
     stage_barrier();
     compute_stage<NRB, SC>(ws0, lds0, sc, col, q, dr, acc);
@@ -874,7 +869,7 @@ int slots() { return 2 * hn_device_cus(); }
 // padding and idle CUs.
 constexpr long kUnits32 = 8192, kUnits64 = 16384;
 
-constexpr long kSplitStages = 32;
+constexpr long kLongK = 64, kSplitStages = 16;
 
 // Where the kernels beside these are faster (us here, theirs; M x N x K, group 128
 // unless said):
@@ -936,7 +931,7 @@ MidPlan mid_plan(int mats, long M, long N, long K, long group) {
   if (T < kShort && (M <= 32 || (M <= 64 && T < kShort / 2))) return p;
   const long nt = (N * mats + kBN - 1) / kBN, tk = kwave_tiles(mats, M, N);
   if (kwave_ok(mats, M, N, T, sps)) {
-    if (mats == 1 && M <= kFewRows && T > 32 && tk < 128 && (tk < 64 || T > 64 || T % kKWaves != 0))
+    if (mats == 1 && M <= kFewRows && T > 32 && tk < 128 && (tk < 64 || T > kLongK || T % kKWaves != 0))
       return p;
     p.kw = p.ok = true;
     p.rbm = 2;
@@ -956,21 +951,23 @@ MidPlan mid_plan(int mats, long M, long N, long K, long group) {
   long lim = hn_device_cus() / tiles;
   if (lim > T / 2) lim = T / 2;
   if (N % 4 != 0) {  // the reduction reads four columns at a time
-    if (T > kSplitStages) return p;
+    if (T > 32) return p;
     lim = 1;
   }
   if (lim < 1 || T < kShort) lim = 1;
   long ks = lim;
   for (long d = lim; d >= 1 && 2 * d >= lim; --d)
     if (T % d == 0) { ks = d; break; }
-  // past K = 8192, splits of at most 32 stages however many tiles there are (us, one
-  // split for each CU and splits of 32: 1500 x 1024 x 14336 96 / 87; gate and up
-  // of 160 x 4096 x 14336 90 / 86)
-  if (T > 2 * kSplitStages) {
-    const long m = (T + kSplitStages - 1) / kSplitStages;
+  // past K = 8192, splits of at most kSplitStages stages, as long as all are resident at
+  // once, an even split where there is one nearby (us by one split per CU / so: 560 x
+  // 1024 x 14336 group 64 65 / 49; 333 x 4096 x 12288 group 64 94 / 74; but up to 64
+  // rows 64 x 8192 x 28672 70 / 82)
+  if (T > kLongK && M > 64) {
+    const long m = std::min((T + kSplitStages - 1) / kSplitStages, std::max(slots() / tiles, 1L));
     long d = m;
-    while (d < 2 * m && T % d != 0) ++d;
-    if (ks < d) ks = T % d == 0 ? d : m;
+    while (4 * d > 3 * m && T % d != 0) --d;
+    if (4 * d <= 3 * m) d = m;
+    if (ks < d) ks = d;
   }
   if (M <= 32 && ks > 1 && mats * N * K < (M <= kFewRows ? kFewWork : kFewWork * 2 / 5)) return p;
   p.ks = (int)ks;
@@ -978,14 +975,13 @@ MidPlan mid_plan(int mats, long M, long N, long K, long group) {
   return p;
 }
 
-// Scales per load: whole vectors when every split of every row starts aligned.
+// Scales per load: whole vectors when every split of every row starts aligned (below
+// group 128 a stage's scales are whole pairs).
 int scale_vec(long K, long ld_s, long group, long ks, const void* s0, const void* s1) {
   const long T = K / kStageK, sps = kStageK / group;
-  if (T % ks == 0) {
-    const long per = T / ks * sps;
-    if (ld_s % 8 == 0 && per % 8 == 0 && aligned16(s0) && aligned16(s1)) return 8;
-    if (ld_s % 2 == 0 && per % 2 == 0 && (((uintptr_t)s0 | (uintptr_t)s1) & 3) == 0) return 2;
-  }
+  const long per = T % ks == 0 ? T / ks * sps : sps;
+  if (ld_s % 8 == 0 && per % 8 == 0 && aligned16(s0) && aligned16(s1)) return 8;
+  if (ld_s % 2 == 0 && per % 2 == 0 && (((uintptr_t)s0 | (uintptr_t)s1) & 3) == 0) return 2;
   return 1;
 }
 

@@ -54,3 +54,14 @@ def test_left_to_the_other_kernels(mats, m, n, k, group, want):
 ])
 def test_few_rows_split_with_work_enough(mats, m, n, k, group, want):
     assert _plan(mats, m, n, k, group) == want
+
+
+@pytest.mark.parametrize("mats,m,n,k,group,want", [
+    (1, 560, 1024, 14336, 64, 7),    # 16 stages each
+    (1, 640, 4096, 11008, 64, 3),    # as many as are resident, though 86 stages go in twos
+    (1, 333, 4096, 14336, 64, 4), (2, 160, 4096, 14336, 64, 4),
+    (1, 1500, 4096, 14336, 64, 0), (1, 64, 8192, 28672, 64, 8), (1, 64, 4096, 14336, 32, 8),
+    (1, 90, 1002, 10240, 64, 0),     # columns not a multiple of 4: no reduction
+])
+def test_long_k_splits(mats, m, n, k, group, want):
+    assert _plan(mats, m, n, k, group) == want
