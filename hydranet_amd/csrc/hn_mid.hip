@@ -901,26 +901,30 @@ long kwave_tiles(int mats, long M, long N) {
 }
 
 // Where mid_kwave_kernel takes a problem: a stage for every wave, the scales of a
-// wave's range in LDS, and a few rounds of workgroups (one per CU), past which its
-// 32-token tiles unpack the weights too often.  us against the kernels below (tiles;
-// M x N x K):
-//   one matrix, 8 - 15 stages, 2 rounds:  448 (200 x 4096 x 1408)    12 /  18
-//                                         832 (400 x 4096 x 1408)    21 /  18
-//   to 64 stages, 5 rounds:              1056 (333 x 6144 x 4096)    44 /  55
-//                                        1568 (200 x 14336 x 4096)   66 /  61
-//   more, 3 rounds:                       704 (333 x 4096 x 14336)   85 /  89
-//   gate and up, 2 rounds (the whole expert): 448 (17 x 14336 x 4096)  58 / 66,
-//     704 (500 x 1408 x 4096) 49 / 49, 896 (37 x 14336 x 4096) 73 / 66,
-//     968 (700 x 1408 x 4096) 67 / 55.
-// Above kKRows rows the gain is small (640 x 4096 x 4096 53 / 58, 1000 x 1408 x 4096
-// 36 / 42) and the reductions across workgroups, which need a workspace and its
-// counters anyway, stay the only path.
-constexpr long kKRows = 480;
+// wave's range in LDS, and up to two rounds of workgroups (one per CU).  Beyond, its
+// 32-token tiles unpack the weights too often, but for one matrix up to three while
+// an XCD's L2 holds the activations, which every 64 weight rows read again; past K =
+// 8192, which the kernel below splits, under two.  us, this kernel and the one below
+// (rounds: M x N x K, group 128 unless said):
+//   1.1: 490 x 1024 x 4096          12 / 27     1.7: 640 x 1408 x 4096          24 / 35
+//   1.9: 700 x 1408 x 4096          23 / 33     1.8: 200 x 4096 x 1408          12 / 18
+//   2.3: 260 x 4096 x 4096          29 / 33     2.3: 850 x 1408 x 4096          36 / 33
+//   2.8: 333 x 4096 x 4096 group 64 32 / 38     2.9: 1500 x 1024 x 4096         40 / 34
+//   2.8: 333 x 4096 x 2048          21 / 20     2.8: the same, group 32         22 / 24
+//   3.3: 400 x 4096 x 4096          40 / 34     3.5: 100 x 14336 x 4096 group 64  41 / 37
+//   1.8: 200 x 4096 x 11008         51 / 60     1.9: 480 x 2048 x 10240         47 / 57
+//   2.0: 1024 x 1024 x 14336        75 / 68     2.4: 600 x 2048 x 11008         73 / 68
+//   gate and up (the whole expert): 1.8: 17 x 14336 x 4096 58 / 66; 2.8: 500 x 1408 x
+//     4096 49 / 49; 3.5: 37 x 14336 x 4096 73 / 66; 3.8: 700 x 1408 x 4096 67 / 55
+constexpr long kL2Bytes = 4 << 20;  // per XCD
 
 bool kwave_ok(int mats, long M, long N, long T, long sps) {
-  const long rounds = mats == 2 || T < 2 * kKWaves ? 2 : T <= 64 ? 5 : 3;
-  return M <= kKRows && T >= kKWaves && (T + kKWaves - 1) / kKWaves * sps <= kKScales &&
-         kwave_tiles(mats, M, N) <= rounds * hn_device_cus();
+  if (T < kKWaves || (T + kKWaves - 1) / kKWaves * sps > kKScales) return false;
+  const long round = hn_device_cus(), tiles = kwave_tiles(mats, M, N);
+  if (T > kLongK) return tiles < 2 * round;
+  if (mats == 1 && M * T * kRowB <= kL2Bytes && (T >= 32 || (T >= 2 * kKWaves && sps > 1)))
+    return tiles <= 3 * round;
+  return tiles <= 2 * round;
 }
 
 MidPlan mid_plan(int mats, long M, long N, long K, long group) {

@@ -1,7 +1,9 @@
 """GPU tests of the split reductions' last-arriver counters (tagged 64-bit
-words, hn_arrive in csrc/hn_common.h) on the two kernels that use them: the
+words, hn_arrive in csrc/hn_common.h) on the three kernels that use them: the
 skinny GEMV's split-K (decode family 1, activations too large for one
-workgroup's LDS) and the prefill GEMM's stream-K.
+workgroup's LDS), the prefill GEMM's stream-K (decode family 1 as well: below a
+few thousand rows the middle-size kernels come first) and the middle-size
+kernels' K splits.
 
 A counter left dirty by a launch stopped part-way is simulated from the host:
 the test writes a count of 3 (tag 0, the value an untagged counter would keep)
@@ -87,7 +89,25 @@ def test_skinny_gate_up_split_k_heals_dirty_counters(family1):
     assert bool(((clean.float() - ref).abs() <= 1e-2 + 2e-3 * ref.abs()).all())
 
 
-def test_stream_k_heals_dirty_counters():
+def test_mid_splits_heal_dirty_counters():
+    M, N, K = 300, 512, 14336  # 10 x 2 tiles of 32 x 256 in 8 splits, a word per wave
+    print(f"[ctr] middle-size split-K M={M} N={N} K={K}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    q, s = g.quantize_int4(torch.randn(N, K, device=DEV, dtype=torch.float16, generator=gen) * 0.02, 64)
+    x = torch.randn(M, K, device=DEV, dtype=torch.float16, generator=gen)
+    clean = g.int4_linear(x, q, s, 64)
+    ctr = _dirty(_lib.gemm_workspace(x.device), SKINNY_CTR_WORDS)
+    again = g.int4_linear(x, q, s, 64)
+    torch.cuda.synchronize()
+    assert torch.equal(again, clean)
+    assert int(ctr[:80].abs().sum()) == 0, "a launch leaves its counters at zero"
+    assert bool((ctr[80:] == 3).all()), "counters the launch did not use are untouched"
+    ctr.zero_()
+    ref = x.float() @ g.dequantize_int4(q, s, 64).float().t()
+    assert bool(((clean.float() - ref).abs() <= 1e-2 + 2e-3 * ref.abs()).all())
+
+
+def test_stream_k_heals_dirty_counters(family1):
     M, N, K = 512, 1024, 4096
     print(f"[ctr] stream-K M={M} N={N} K={K}", flush=True)
     x, q, s = _operands(M, N, K, 4)

@@ -65,3 +65,21 @@ def test_few_rows_split_with_work_enough(mats, m, n, k, group, want):
 ])
 def test_long_k_splits(mats, m, n, k, group, want):
     assert _plan(mats, m, n, k, group) == want
+
+
+@pytest.mark.parametrize("mats,m,n,k,group,want", [
+    # over a workgroup's waves: up to two rounds of 256 tiles of 32 x 64 at any number of rows
+    (1, 512, 1024, 4096, 128, -1), (1, 700, 1408, 4096, 128, -1), (1, 2048, 512, 4096, 128, -1),
+    (1, 4096, 256, 1024, 32, -1), (1, 850, 1408, 4096, 128, 1), (1, 200, 4096, 1408, 128, -1),
+    (1, 400, 4096, 1408, 128, 1),
+    # up to three with the activations in L2, at group 128 from 32 stages on
+    (1, 333, 4096, 4096, 128, -1), (1, 333, 4096, 4096, 64, -1), (1, 400, 4096, 4096, 128, 1),
+    (1, 1500, 1024, 4096, 128, 1), (1, 333, 4096, 2048, 64, -1), (1, 333, 4096, 2048, 128, 1),
+    # under two past K = 8192
+    (1, 260, 1024, 14336, 128, -1), (1, 200, 4096, 14336, 128, -1), (1, 225, 4096, 14336, 128, 7),
+    (1, 480, 2048, 10240, 128, -1),
+    (1, 333, 4096, 14336, 128, 4),
+    (2, 333, 1408, 4096, 128, -1), (2, 500, 1408, 4096, 128, 1),
+])
+def test_k_over_waves(mats, m, n, k, group, want):
+    assert _plan(mats, m, n, k, group) == want
