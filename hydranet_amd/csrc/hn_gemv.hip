@@ -683,16 +683,21 @@ static int mid_down_split(long E, long rows, long H, long I, long group) {
              ? kHnDownSplit : 0;
 }
 
+static long mid_down_bytes(long rows, long H) {
+  return (long)kCtrRegion + (long)kHnDownSplit * rows * H * 4;
+}
+
+// (Slices past the prefill workspace, which every caller above 64 tokens has, are left
+// to the prefill GEMM whatever the size of the buffer that is passed: the route,
+// and with it the last bits, follow from the sizes alone.)
 static bool mid_grouped_ok(long E, long max_rows, long rows, long H, long I, long group) {
   if (g_decode_path != 0 || max_rows <= kStreamMaxRows || rows > kMidAvgRows * E) return false;
   if (max_rows <= kMaxRows && rows <= kStreamAvgRows * E) return false;
-  return hn_mid_grouped_impl(0, nullptr, H, nullptr, nullptr, nullptr, nullptr, E, rows, H, I,
-                             group, nullptr, I, nullptr, 1, nullptr, 1) == 0 &&
-         mid_down_split(E, rows, H, I, group) != 0;
-}
-
-static long mid_down_bytes(long rows, long H) {
-  return (long)kCtrRegion + (long)kHnDownSplit * rows * H * 4;
+  if (hn_mid_grouped_impl(0, nullptr, H, nullptr, nullptr, nullptr, nullptr, E, rows, H, I,
+                          group, nullptr, I, nullptr, 1, nullptr, 1) != 0)
+    return false;
+  const int ks = mid_down_split(E, rows, H, I, group);
+  return ks == 1 || (ks != 0 && mid_down_bytes(rows, H) <= hn_gemm_workspace_bytes());
 }
 
 extern "C" int hn_set_decode_path(int path) {

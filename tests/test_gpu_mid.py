@@ -131,6 +131,26 @@ def test_experts_uneven(e, h, i, tokens, k):
     _close(out / k, ref / k)
 
 
+def test_route_ignores_the_size_of_the_workspace():
+    """16384 rows of 512 columns in four fp32 slices are more than the prefill workspace
+    holds; a larger buffer left by another call changes neither the kernel nor a bit."""
+    table = moe.ExpertTable.from_slots(_layer(128, 512, 4608, 3))
+    gen = torch.Generator().manual_seed(4)
+    idx = torch.randint(0, 128, (8192, 2), generator=gen, dtype=torch.int32).cuda()
+    w = torch.rand(8192, 2, generator=gen).half().cuda()
+    x = _x(8192, 512, 8)
+    kept = dict(_lib._WORKSPACES)
+    try:
+        _lib._WORKSPACES.clear()
+        want = moe.moe_experts_forward(x, idx, w, table)
+        _lib.workspace(160 << 20, x.device)
+        assert torch.equal(moe.moe_experts_forward(x, idx, w, table), want)
+    finally:
+        torch.cuda.synchronize()
+        _lib._WORKSPACES.clear()
+        _lib._WORKSPACES.update(kept)
+
+
 @pytest.mark.parametrize("t,k,i", [(96, 2, 2048), (96, 2, 6144), (33, 4, 2048)])
 def test_layer_graph_replay(t, k, i):
     """The layer's launches captured once and replayed: every replay as the eager run."""

@@ -83,3 +83,26 @@ def test_long_k_splits(mats, m, n, k, group, want):
 ])
 def test_k_over_waves(mats, m, n, k, group, want):
     assert _plan(mats, m, n, k, group) == want
+
+
+@pytest.mark.parametrize("e,rows,h,i,split", [
+    (8, 1024, 4096, 14336, True), (128, 16000, 4096, 1408, False),
+    (32, 2000, 4096, 6144, True), (32, 3000, 4096, 6144, False), (128, 16384, 512, 4608, False),
+])
+def test_down_slices_fit_the_prefill_workspace(e, rows, h, i, split):
+    """Whether a layer's down projection runs in K slices follows from its sizes: where it
+    does, the slices fit the workspace that every caller above 64 tokens passes."""
+    lib = _lib.lib()
+    got = lib.hn_moe_experts_decode_split_check(e, rows, rows, h, i, 128) == 0
+    assert got == split
+    if got:
+        assert (2 << 20) + 16 * rows * h <= lib.hn_gemm_workspace_bytes()
+
+
+def test_product_splits_fit_the_prefill_workspace():
+    ws = _lib.lib().hn_gemm_workspace_bytes()
+    for mats in (1, 2):
+        for m in (65, 100, 333, 560, 1024, 1500, 2048, 4096, 8192):
+            for n in (64, 256, 1000, 4096, 14336, 32000):
+                for k in (1024, 1408, 4096, 8192, 14336, 28672):
+                    assert (2 << 20) + _part_bytes(mats, m, n, k) <= ws, (mats, m, n, k)
