@@ -226,7 +226,8 @@ struct TileLoads {
   const void* px; int nx;             // activation rows of the tile, bytes
   const void* pq[kBlk];               // packed weights of each block's matrix
   const void* ps[kBlk];               // scales
-  int nq, ns;                         // bytes of one packed / scale matrix (ns: whole dwords)
+  int nq;                             // bytes of one packed matrix
+  int ns[kBlk];                       // bytes of scales from ps to the last one, whole dwords
   uint32_t va[kALoadsMax];            // activation chunk offsets (first a_loads<NRB>)
   uint32_t vq[kBlk];                  // weight byte offset of (lane's row, lane's 16 B)
   uint32_t vs[kBlk];                  // scale byte offset of the lane's row
@@ -246,10 +247,11 @@ __device__ __forceinline__ uint32_t a_offset(int j, int wave, int lane, int rows
 }
 
 // Byte offset of the 16 bytes holding groups g .. g + 3 (g a multiple of 4) of
-// the row whose scales start at byte row: the dword of group g, moved back
-// where 16 bytes would end past the matrix.
-__device__ __forceinline__ uint32_t scale_src(const TileLoads& tl, uint32_t row, int g) {
-  return min((row + 2 * g) & ~3u, (uint32_t)tl.ns - 16);
+// the row of block b: the dword of group g, moved back where 16 bytes would end
+// past the matrix.  ps is a dword's address (vs holds the half word that a row may
+// start on), so the dword of the last scale is the furthest byte read.
+__device__ __forceinline__ uint32_t scale_src(const TileLoads& tl, int b, int g) {
+  return min((tl.vs[b] + 2 * g) & ~3u, (uint32_t)tl.ns[b] - 16);
 }
 
 // Issue stage t's loads into the LDS stage at byte address st, and those of
@@ -270,7 +272,7 @@ __device__ __forceinline__ void issue_stage(const TileLoads& tl, int t, int grp,
   if (real && grp % kScRun == 0 && grp * tl.group == kKS * t) {  // uniform
 #pragma unroll
     for (int b = 0; b < kBlk; ++b)
-      dma_b128(rsrc(tl.ps[b], tl.ns), scale_src(tl, tl.vs[b], grp + 4 * h), 0,
+      dma_b128(rsrc(tl.ps[b], tl.ns[b]), scale_src(tl, b, grp + 4 * h), 0,
                sc0 + (grp / kScRun & 1) * kScSlot + (wave * kBlk + b) * 1024);
   }
   {
@@ -365,7 +367,7 @@ __device__ __forceinline__ void read_b(Ops& o, const TileLoads& tl, uint32_t st,
       for (int i = 0; i < 4; ++i) o.pk[b][4 * d + i] = v[i];
     }
     o.sv[b] = lds_read<unsigned short>(slot + (wave * kBlk + b) * 1024 + tl.vs[b] + 2 * g -
-                                       scale_src(tl, tl.vs[b], g & ~3));
+                                       scale_src(tl, b, g & ~3));
   }
 }
 
@@ -823,17 +825,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kOccW, kOcc
     tl.px = pr.x + (long)m0 * A.ld_x + k0;
     tl.nx = (int)(rows * A.ld_x * 2 - 2 * k0);
     tl.nq = N * A.ld_q - k0 / 2;
-    tl.ns = ((N * A.ld_s - k0 / A.group) * 2 + 3) & ~3;
+    const int n_sc = (N - 1) * A.ld_s + (A.K - k0) / A.group;  // scales from here to the last
     tl.group = A.group;
 #pragma unroll
     for (int b = 0; b < kBlk; ++b) {
       const int mt = MATS == 2 ? b : 0;
       const int row = MATS == 2 ? n0 : n0 + 32 * b;
       tl.pq[b] = pr.q[mt] + k0 / 2;
-      tl.ps[b] = pr.s[mt] + k0 / A.group;
+      const uintptr_t ps = (uintptr_t)(pr.s[mt] + k0 / A.group);
+      const int odd = (int)(ps & 2);  // scales may start on any half word
+      tl.ps[b] = (const void*)(ps - odd);
+      tl.ns[b] = (odd + 2 * n_sc + 3) & ~3;
       const bool ok = row < N;
       tl.vq[b] = ok ? (uint32_t)(row * A.ld_q + 16 * kKSM * h) : kOOB;
-      tl.vs[b] = (uint32_t)(2 * min(row, N - 1) * A.ld_s);
+      tl.vs[b] = (uint32_t)(odd + 2 * min(row, N - 1) * A.ld_s);
     }
     f32x16 acc[kRBMax][kBlk];
 #pragma unroll

@@ -11,7 +11,6 @@ import torch
 import oracle
 from hydranet_amd import _lib
 
-pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 L, P = ctypes.c_long, ctypes.c_void_p
 
@@ -26,6 +25,7 @@ def _gemm(x, p, s, out, N, K, g, work):
              None if work is None else work.data_ptr(), 0 if work is None else work.numel(), st)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,g,pad", [
     (65, 9, 128, 128, 0),       # 18 bytes of scales in all
     (70, 33, 11 * 128, 128, 0), # odd row stride, a run and three groups
@@ -55,3 +55,54 @@ def test_gemm_scale_runs(M, N, K, g, pad):
         bound = 2 * K * 2.0 ** -24 * size + 2.0 ** -10 * ref.abs() + 1e-6
         err = (out.float() - ref).abs()
         assert bool((err <= bound).all()), float((err / bound).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,g", [(65, 33, 11 * 128, 128), (130, 300, 17 * 128, 128),
+                                     (66, 101, 9 * 64, 64), (65, 41, 320, 32), (257, 520, 4096, 128)])
+@pytest.mark.parametrize("view", ["odd", "right"])
+def test_gemm_scales_of_a_view(M, N, K, g, view):
+    """Scales that start on the second half of a dword, and scales that are the last
+    columns of a wider matrix (whose last row ends where the memory does)."""
+    print(f"[scales] {view} M={M} N={N} K={K} g={g}", flush=True)
+    gen = torch.Generator().manual_seed(M + K)
+    w = (torch.randn(N, K, generator=gen) * 0.02).half()
+    w *= (2.0 ** (torch.arange(K // g) * 5 % 7 - 3)).repeat_interleave(g).half()
+    x = torch.randn(M, K, generator=gen).half().to(DEV)
+    q, sc = oracle.quantize(w.numpy(), g, mode=0)
+    deq = torch.from_numpy(oracle.dequant(q, sc, g).astype(np.float32)).to(DEV)
+    p, kg = torch.from_numpy(q).to(DEV), K // g
+    if view == "odd":
+        s = torch.full((N * kg + 1,), float("nan"), dtype=torch.float16, device=DEV)[1:].view(N, kg)
+        assert s.data_ptr() % 4 == 2
+    else:
+        s = torch.full((N, kg + 9), float("nan"), dtype=torch.float16, device=DEV)[:, 9:]
+    s.copy_(torch.from_numpy(sc.copy()))
+    ref = x.float() @ deq.t()
+    bound = 2 * K * 2.0 ** -24 * (x.float().abs() @ deq.abs().t()) + 2.0 ** -10 * ref.abs() + 1e-6
+    for work in (None, _lib.gemm_workspace(DEV)):
+        out = torch.full((M, N), 7.0, dtype=torch.float16, device=DEV)
+        assert _gemm(x, p, s, out, N, K, g, work) == 0
+        assert bool(((out.float() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("ld_s,kg,odd", [(1, 1, 0), (1, 1, 2), (3, 3, 2), (11, 11, 0), (11, 11, 2),
+                                         (40, 31, 0), (40, 31, 2), (32, 32, 2)])
+@pytest.mark.parametrize("N", [9, 33, 100])
+def test_scale_loads_stay_in_the_matrix(ld_s, kg, odd, N):
+    """The byte ranges of the kernel's scale loads (its own arithmetic, on the host): every
+    16 bytes from the dword of the first scale to the dword of the last, every scale that is
+    read back inside what was loaded for it, whole tiles and later segments."""
+    for first in range(0, kg, 2):                      # a segment's first group
+        addr = 64 + odd + 2 * first                    # of the segment's first scale
+        base = addr & ~3
+        end = odd + 64 + 2 * ((N - 1) * ld_s + kg)     # past the last scale
+        ns = ((addr & 2) + 2 * ((N - 1) * ld_s + kg - first) + 3) & ~3
+        if ns < 16:
+            continue                                   # not taken
+        for row in {0, 1, N // 2, N - 2, N - 1}:
+            vs = (addr & 2) + 2 * row * ld_s
+            for g in range(kg - first):
+                src = min((vs + 2 * (g & ~3)) & ~3, ns - 16)
+                assert (64 + odd) & ~3 <= base + src and base + src + 16 <= (end + 3) & ~3
+                assert 0 <= vs + 2 * g - src <= 14
