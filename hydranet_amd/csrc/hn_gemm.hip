@@ -246,6 +246,10 @@ __device__ __forceinline__ uint32_t a_offset(int j, int wave, int lane, int rows
   return (uint32_t)((min(r, rows - 1) * (int)ld_x + 8 * c) * 2);
 }
 
+// Fewest scales, from a tile's or segment's first to the matrix's last, that 16 bytes
+// of whole dwords lie within.
+constexpr long kMinScales = 7;
+
 // Byte offset of the 16 bytes holding groups g .. g + 3 (g a multiple of 4) of
 // the row of block b: the dword of group g, moved back where 16 bytes would end
 // past the matrix.  ps is a dword's address (vs holds the half word that a row may
@@ -926,6 +930,7 @@ bool sk_setup(GemmArgs& A, void* work, long work_bytes, long tiles_upper, dim3& 
   const int g = kOcc * num_cus();
   if (!work || work_bytes < sk_bytes() || tiles_upper * kWaves > kSkCounters || g > kSkMaxGrid)
     return false;
+  if ((A.N - 1L) * A.ld_s + 1 < kMinScales) return false;  // a segment may start with the last
   // chunk: the largest divisor of the stages per tile up to 16 whose k span
   // is an even number of scale groups (segment pointers then move by whole
   // scale dwords)
@@ -949,13 +954,12 @@ bool sk_setup(GemmArgs& A, void* work, long work_bytes, long tiles_upper, dim3& 
 // Shape checks shared by the entry points below: 1 when the GEMM kernels
 // handle the shape.
 static int gemm_shape_ok(long N, long K, long group, long ld_q, long ld_s) {
-  // a lane's 32 kKSM k of a stage share one scale, and the scale offset split
-  // (voffset: lane part, soffset: stage part) needs group 32 kKSM or a
-  // multiple of the stage
+  // a lane's 32 kKSM k of a stage share one scale: group 32 kKSM or a multiple of
+  // the stage
   if (K <= 0 || K % kKS != 0 || group <= 0 || K % group != 0) return 0;
   if (group != 32 * kKSM && group % kKS != 0) return 0;
   if (ld_q % 16 != 0) return 0;
-  if (N <= 8) return 0;  // at least 16 bytes of scales (scale_src)
+  if ((N - 1) * ld_s + K / group < kMinScales) return 0;
   if (N * ld_q >= (long)kOOB || N * ld_s * 2 >= (long)kOOB) return 0;
   return 1;
 }

@@ -744,8 +744,15 @@ static int run_single(int mats, const void* x, long ld_x, W4Mat w0, W4Mat w1, vo
     if (rc != HN_NOT_HANDLED) return rc;
   }
   const int tiles = hn_cdiv(N, kTileN);
-  for (long m0 = 0; m0 < M; m0 += kMaxRows) {
-    const int rows = (int)((M - m0) > kMaxRows ? kMaxRows : (M - m0));
+  // above kMaxRows rows no workspace is asked for: the few products with a handful of
+  // scales in all, which the GEMM does not take, run in chunks of rows that need none
+  long step = kMaxRows;
+  if (M > kMaxRows && (N - 1) * w0.ld_s + K / group < 8 &&
+      (!ws || (size_t)ws_size < ctr_bytes(tiles) + part_bytes(make_plan(kMaxRows, (int)K, mats).ks,
+                                                              mats, kMaxRows, N)))
+    while (step > 1 && make_plan((int)step, (int)K, mats).ks > 1) step /= 2;
+  for (long m0 = 0; m0 < M; m0 += step) {
+    const int rows = (int)((M - m0) > step ? step : (M - m0));
     const Plan p = make_plan(rows, (int)K, mats);
     HN_ARG_CHECK((n_counters < tiles ? tiles : n_counters) <= kMaxCounters,
                  "%s: N=%ld needs more split-K counters than the workspace holds", who, N);

@@ -106,3 +106,36 @@ def test_scale_loads_stay_in_the_matrix(ld_s, kg, odd, N):
                 src = min((vs + 2 * (g & ~3)) & ~3, ns - 16)
                 assert (64 + odd) & ~3 <= base + src and base + src + 16 <= (end + 3) & ~3
                 assert 0 <= vs + 2 * g - src <= 14
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mats", [1, 2])
+@pytest.mark.parametrize("M,N,K,g", [
+    (1000, 8, 10240, 512), (70, 1, 4096, 4096), (300, 2, 8192, 4096), (65, 6, 4096, 4096),
+    (130, 7, 4096, 4096), (200, 1, 10240, 512), (66, 3, 2048, 1024), (100, 8, 4096, 128),
+])
+def test_few_scales_need_no_workspace(M, N, K, g, mats):
+    """More than 64 rows of a product with few columns and a handful of scales, with no
+    workspace and with the prefill one."""
+    print(f"[scales] few M={M} N={N} K={K} g={g} mats={mats}", flush=True)
+    gen = torch.Generator().manual_seed(M + K)
+    x = (torch.randn(M, K, generator=gen) * 0.25).half().to(DEV)
+    deq, ptrs = [], []
+    for _ in range(mats):
+        q, sc = oracle.quantize((torch.randn(N, K, generator=gen) * 0.02).half().numpy(), g, mode=0)
+        deq.append(torch.from_numpy(oracle.dequant(q, sc, g).astype(np.float32)).to(DEV))
+        ptrs += [torch.from_numpy(q).to(DEV), torch.from_numpy(sc.copy()).to(DEV)]
+    prod = [x.float() @ d.t() for d in deq]
+    ref = prod[0] if mats == 1 else torch.nn.functional.silu(prod[0].half().float()) * prod[1].half().float()
+    for work in (None, _lib.gemm_workspace(DEV)):
+        out = torch.full((M, N), 7.0, dtype=torch.float16, device=DEV)
+        tail = (_lib.ptr(out), N, M, N, K, g, _lib.ptr(work), 0 if work is None else work.numel(),
+                _lib.stream())
+        if mats == 1:
+            _lib.call("hn_int4_linear", _lib.ptr(x), K, _lib.ptr(ptrs[0]), K // 2, _lib.ptr(ptrs[1]),
+                      K // g, *tail)
+        else:
+            _lib.call("hn_int4_gate_up_silu", _lib.ptr(x), K, *[_lib.ptr(t) for t in ptrs], K // 2,
+                      K // g, *tail)
+        # the repository's bar for fp16 outputs
+        assert bool(((out.float() - ref).abs() <= 1e-2 + 2e-3 * ref.abs()).all())
