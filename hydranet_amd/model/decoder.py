@@ -148,9 +148,11 @@ class Attention(nn.Module):
                 and (mask is None or (mask.dtype == torch.float16 and mask.numel() == kv_len
                                       and mask.is_contiguous())))
 
-    def _prefill_fits(self, x: torch.Tensor, S: int, cache: "KVCache", kv_len: int,
+    def _prefill_fits(self, x: torch.Tensor, S: int, cache: "KVCache", layer: int, kv_len: int,
                       mask: Optional[torch.Tensor]) -> bool:
-        """The one-kernel form walks a workgroup's positions one tile of 64
+        """Whether the one-kernel form (raw pointers) takes this call; a cache or mask
+        that is not laid out for x is left to the products, which say what is wrong
+        with it.  The one-kernel form walks a workgroup's positions one tile of 64
         after the other (about 1.9 us each); the two products spread a long
         past over the chip.  Their times cross where there are about as many
         workgroups as tiles (B, S, past: one kernel / products, us, whole
@@ -160,11 +162,16 @@ class Attention(nn.Module):
         rep = self.nh // self.nkv
         rows = S * rep if S < 128 else S  # see hn_attn_prefill: heads share a tile below 128
         wgs = x.shape[0] * self.nh * S // rows * -(-rows // 128)
+        kt, v = cache.kt[layer], cache.v[layer]
         return (self.decode_kernel and x.is_cuda and S > 1 and self.hd == 128
                 and 8 * wgs >= 7 * -(-kv_len // 64)
                 and cache.max_len % 8 == 0 and 1 <= kv_len <= cache.max_len < 1 << 22
                 and rep * S < 1 << 22
-                and (mask is None or (mask.dtype == torch.float16 and mask.is_cuda
+                and tuple(kt.shape) == (x.shape[0], self.nkv, self.hd, cache.max_len)
+                and tuple(v.shape) == (x.shape[0], self.nkv, cache.max_len, self.hd)
+                and all(t.dtype == torch.float16 and t.device == x.device and t.is_contiguous()
+                        for t in (kt, v))
+                and (mask is None or (mask.dtype == torch.float16 and mask.device == x.device
                                       and tuple(mask.shape) == (S, kv_len)
                                       and mask.stride(1) == 1 and mask.stride(0) >= kv_len)))
 
@@ -249,7 +256,7 @@ class Attention(nn.Module):
                       _lib.ptr(cache.v[layer]), cache.max_len, B, nkv, rep, hd, kv_len,
                       _lib.ptr(mask), inv, _lib.ptr(o), o.stride(0), _lib.stream(x.device))
             return self.o_proj(o.view(B, S, nh * hd))
-        if self._prefill_fits(x, S, cache, kv_len, mask):
+        if self._prefill_fits(x, S, cache, layer, kv_len, mask):
             from .. import _lib
             o = torch.empty((B * S, nh * hd), dtype=x.dtype, device=x.device)
             work = None

@@ -7,6 +7,7 @@ form), grouped-query attention equals textbook per-head attention with KV head
 h // (heads / kv_heads), and RoPE preserves norms and is relative
 (q(m) . k(n) depends on m - n only)."""
 import math
+import types
 
 import torch
 
@@ -134,3 +135,25 @@ def test_kv_cache_bounds():
         pass
     else:
         raise AssertionError("advance past max_len must fail")
+
+
+def test_prefill_kernel_takes_only_its_own_cache():
+    """The one-kernel form reads by raw pointers: a cache of another batch, type or head
+    count, or a mask of another shape, stays with the products (which refuse it)."""
+    cfg = MixtralDecoderConfig(num_layers=1, hidden_dim=512, num_attention_heads=4, num_kv_heads=2)
+    att = Attention(cfg).half()
+    B, S, L = 2, 130, 256
+    x = types.SimpleNamespace(is_cuda=True, shape=(B, S, 512), device=torch.device("cpu"))
+
+    def fits(batch=B, nkv=2, hd=128, dtype=torch.float16, mask=None, strided=False):
+        cache = KVCache(1, batch, nkv, hd, L, "cpu", dtype)
+        if strided:
+            cache.kt[0] = cache.kt[0].transpose(2, 3).contiguous().transpose(2, 3)
+        return att._prefill_fits(x, S, cache, 0, S, mask)
+
+    half = causal_mask(0, S, "cpu", torch.float16)
+    assert fits() and fits(mask=half)
+    assert not fits(batch=1) and not fits(batch=4) and not fits(nkv=4) and not fits(hd=64)
+    assert not fits(dtype=torch.float32) and not fits(dtype=torch.bfloat16) and not fits(strided=True)
+    assert not fits(mask=half.float()) and not fits(mask=half[:, :-1]) and not fits(mask=half[None])
+    assert not fits(mask=half.to("meta"))

@@ -160,6 +160,22 @@ def test_attention_module_routes_agree(S, L, masked):
     assert rel.item() < 2e-3, rel.item()
 
 
+@pytest.mark.parametrize("batch,dtype", [(4, torch.float16), (2, torch.float32)])
+def test_attention_module_refuses_another_cache(batch, dtype):
+    """Two sequences against a cache of four, or of fp32: an error, as by the products."""
+    from hydranet_amd.model.decoder import Attention, KVCache, MixtralDecoderConfig, RotaryEmbedding
+    cfg = MixtralDecoderConfig(hidden_dim=512, num_attention_heads=4, num_kv_heads=2)
+    att = Attention(cfg).half().to(DEV)
+    rope = RotaryEmbedding(HD, 256, 1e6, device=DEV)
+    x = torch.randn(2, 130, 512, device=DEV).half()
+    for on in (True, False):
+        att.decode_kernel = on
+        cache = KVCache(1, batch, 2, HD, 256, DEV, dtype)
+        with pytest.raises(RuntimeError):
+            with torch.no_grad():
+                att(x, rope, torch.arange(130, device=DEV), cache, 0, 130, _causal(130, 130))
+
+
 @pytest.mark.parametrize("B,S,nh,nkv", [(2, 8, 8, 2), (1, 63, 4, 1), (2, 65, 12, 3), (1, 333, 32, 8)])
 def test_rope_append_runs_equal_elementwise(B, S, nh, nkv):
     """The kernel for runs of tokens against the one-element kernel (taken when
