@@ -1028,10 +1028,10 @@ constexpr long kRows32 = 20;
 }  // namespace
 
 // How a single problem is run here: 0 not at all, -1 K over the waves of a workgroup,
-// else the number of K splits over workgroups (1: whole).
+// else the tile's tokens << 16 | the number of K splits over workgroups (1: whole).
 extern "C" int hn_mid_linear_plan(int mats, long M, long N, long K, long group) {
   const MidPlan p = mid_plan(mats, M, N, K, group);
-  return !p.ok ? 0 : p.kw ? -1 : p.ks;
+  return !p.ok ? 0 : p.kw ? -1 : p.rbm << 20 | p.ks;
 }
 
 // Workspace bytes (after kPartOffset) a single problem's K splits need; 0 when

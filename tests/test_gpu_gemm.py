@@ -1,5 +1,7 @@
-"""GPU parity of the prefill MFMA GEMM path (more than 64 tokens per weight
-matrix): hn_int4_linear, hn_expert_mlp_int4 and the grouped MoE dispatch.
+"""GPU parity above 64 tokens per weight matrix: hn_int4_linear,
+hn_expert_mlp_int4 and the grouped MoE dispatch, each by the prefill MFMA GEMM
+(decode family 1 keeps the middle-size kernels out) and by whichever kernels the
+sizes are given to.
 
 References: the CPU oracle (oracle.int4_linear, torch_ref.expert_mlp,
 torch_ref.moe_dispatch) where it finishes in seconds, and at full Mixtral
@@ -29,6 +31,14 @@ def _no_tf32():
     torch.backends.cuda.matmul.allow_tf32 = False
     yield
     torch.backends.cuda.matmul.allow_tf32 = old
+
+
+@pytest.fixture(autouse=True, params=[1, 0], ids=["gemm", "auto"])
+def _kernels(request):
+    from hydranet_amd import _lib
+    _lib.set_decode_path(request.param)
+    yield
+    _lib.set_decode_path(0)
 
 
 def _rand_f16(seed, shape, scale=1.0):

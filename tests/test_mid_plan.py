@@ -17,7 +17,8 @@ def _plan(mats, m, n, k, group):
     """0: not a product for these kernels; -1: K over a workgroup's waves; else K splits."""
     f = _lib.lib().hn_mid_linear_plan
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_int] + [ctypes.c_long] * 4
-    return f(mats, m, n, k, group)
+    r = f(mats, m, n, k, group)
+    return r if r <= 0 else r & 0xffff
 
 
 @pytest.mark.parametrize("mats,m,n,k", [(1, 1500, 4096, 4096), (1, 1024, 6144, 4096),
