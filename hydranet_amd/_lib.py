@@ -78,8 +78,9 @@ RESTYPES = {"hn_skinny_workspace_bytes": ctypes.c_long,
             "hn_attn_prefill_workspace_bytes": ctypes.c_long, "hn_gemm_workspace_bytes": ctypes.c_long,
             "hn_moe_decode_layer_partials": ctypes.c_long}
 
-# Tokens per weight matrix up to which the decode (skinny / streaming) kernels
-# run; above it the MFMA GEMM kernels do (kMaxRows in csrc/hn_gemv.hip).
+# Tokens per weight matrix up to which the decode (skinny / streaming) kernels run
+# where the middle-size kernels do not (from 17 on); above it the MFMA GEMM kernels do
+# (kMaxRows in csrc/hn_gemv.hip), and a call passes the GEMM's workspace.
 DECODE_MAX_ROWS = 64
 
 _lib = None
@@ -114,8 +115,8 @@ _DECODE_PATH = threading.local()
 
 
 def set_decode_path(path: int) -> None:
-    """Decode kernel family of the calling thread: 0 = the streaming kernels
-    where they apply, 1 = split-K kernels only (A/B measurement and tests)."""
+    """Kernel family of the calling thread: 0 = by size, 1 = the split-K kernels up to
+    64 rows and the prefill GEMM above only (A/B measurement and tests)."""
     call("hn_set_decode_path", path)
     _DECODE_PATH.value = path
 
@@ -160,7 +161,8 @@ def skinny_workspace(kind: int, M: int, N: int, K: int, E: int, device) -> torch
 
 
 def gemm_workspace(device) -> torch.Tensor:
-    """Workspace of the prefill GEMM kernels' stream-K split (about 128 MiB)."""
+    """Workspace above DECODE_MAX_ROWS tokens: the prefill GEMM's stream-K split and the
+    middle-size kernels' K splits (about 128 MiB)."""
     return workspace(lib().hn_gemm_workspace_bytes(), device)
 
 

@@ -153,9 +153,10 @@ __device__ __forceinline__ void wait_vmcnt() {
 // their side of it, and the loads of later stages stay in flight.  (A
 // __syncthreads is also a release fence, for which the compiler waits until
 // every LDS-DMA load of the wave has landed: the loads of stage t + 2, issued
-// at the start of stage t, then had to arrive before stage t could end.
-// Mixtral layer on MI355X with the one and the other: 2048 tokens 1805 ->
-// 1692 us, 100 tokens 561 -> 482 us.)
+// at the start of stage t, then had to arrive before stage t could end.  4096
+// rows over eight Mixtral experts on MI355X, with __syncthreads and with this: 1571
+// to 102 rows each, gate/up 1012 -> 994 us, down 548 -> 536; 512 each, 877 -> 872 and
+// 428 -> 424.)
 __device__ __forceinline__ void stage_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
@@ -203,8 +204,8 @@ struct Stage {
 // as for 16 bytes, 65 cycles, so loading each stage's scale dwords anew took 520
 // cycles of the CU's path per stage, next to 1350 for activations and weights
 // and 2048 for the stage's MFMAs.  4096 rows over eight Mixtral experts on
-// MI355X, per-stage dwords and runs: gate/up 991 -> 979 us, down 511 -> 483 us;
-// the layer of 2048 tokens 1725 -> 1700 us.)
+// MI355X, per-stage dwords and runs: 1571 to 102 rows each, gate/up 995 -> 994 us,
+// down 554 -> 536; 512 each, 880 -> 872 and 461 -> 424.)
 constexpr int kScRun = 8;
 constexpr int kScSlot = kWaves * kBlk * 1024;  // bytes
 constexpr int kLdsBytes = kNST * Stage::kSize + 2 * kScSlot;

@@ -649,30 +649,36 @@ extern "C" int hn_gemm_grouped_impl(int phase, const void* x, long ld_x, const v
                                     long ld_o, void* work, long work_bytes, void* stream);
 extern "C" long hn_gemm_workspace_bytes();
 
-// Decode kernel family: 0 = automatic (streaming kernels where they apply),
-// 1 = split-K kernels only.  Per calling thread (a switch in one thread never
+// Kernel family: 0 = automatic (streaming, middle-size, split-K, prefill GEMM),
+// 1 = split-K kernels, and the prefill GEMM above 64 rows, only.  Per calling thread (a switch in one thread never
 // changes another thread's calls); for A/B measurement and tests.
 static thread_local int g_decode_path = 0;
 
 // Which kernels take a grouped launch of group 128.  Up to 16 rows per expert the
 // streaming kernels do, in one pass over the weights; past that by the average:
 //  * up to 10 rows per expert the streaming kernels (passes of 8 or 16 tokens of
-//    whole K, at most 64 rows): us gate/up + down, 8 experts of 4096 x 14336,
-//    8 rows each 95 + 50 against 111 + 61 by the middle-size kernels; 12 rows
-//    113 + 67 against 113 + 62;
-//  * up to 128 rows the middle-size kernels (hn_mid.hip): 24 rows each 129 + 66
-//    against 241 + 126 by the prefill GEMM, 128 rows 310 + 155 against 319 + 163;
-//    128 experts of 4096 x 1408, 32 rows 196 + 122 against 367 + 237.  Above 64
-//    rows for one expert they also take the smaller averages, where the
-//    streaming kernels' bound on an expert's rows does not hold;
+//    whole K, at most 64 rows).  us, both phases and the unpermute, 8 experts of 4096 x
+//    14336, by them / by the middle-size kernels, each of several sampled routings
+//    (uniform; Zipf popularity): average 6 158-168 / 174 and 158-168 / 172; 8 168-170 /
+//    175 and 161-195 / 171-183; 10 171-195 / 175-182 and 215 / 185; 12 199 / 183 and
+//    217 / 179.  128 experts of 4096 x 1408, average 4: 232-244 / 272 and 168 / 164;
+//  * up to 128 rows the middle-size kernels (hn_mid.hip; hidden sizes up to 4096,
+//    intermediate ones up to 4096 whole and 16384 in K slices: larger layers have not
+//    been measured and keep the other two).  us as above, by the prefill GEMM / by them: average 25
+//    434 / 222 and 451 / 262; 75 511 / 400 and 538 / 404; 128 609 / 587 and 662 / 585;
+//    128 experts, 31 728 / 375 and 651 / 381; 128 1045 / 895 and 1167 / 934.  Above 64
+//    rows for one expert they also take the smaller averages, where the streaming
+//    kernels' bound on an expert's rows does not hold.  The average is over all experts:
+//    with every token on the same two of 8 experts of 512 rows they take 473 us, the
+//    GEMM 432;
 //  * above, the prefill GEMM (192 rows each 410 + 230 against 447 + 233).
 constexpr long kStreamAvgRows = 10, kMidAvgRows = 128;
 static bool stream_rows_ok(long max_rows, long rows, long E) {
   return max_rows <= kStreamMaxRows || (max_rows <= kMaxRows && rows <= 16 * E);
 }
 
-// K slices of the middle-size kernels' down projection: whole where a row's
-// scales fit their LDS copy, else the split the unpermute sums (0: neither).
+// K slices of the middle-size kernels' down projection: whole up to 4096 k, else the
+// split that the unpermute sums (0: neither).
 static int mid_down_split(long E, long rows, long H, long I, long group) {
   static float dummy;
   if (hn_mid_grouped_impl(1, nullptr, I, nullptr, nullptr, nullptr, nullptr, E, rows, H, I, group,
@@ -853,7 +859,7 @@ extern "C" int hn_silu_then_mul(const void* g, long ld_g, const void* u, long ld
   return 0;
 }
 
-// Grouped decode over one MoE layer (<= 64 rows per expert).
+// Grouped SwiGLU over one MoE layer.
 //   x_perm [rows, H] fp16 sorted by expert; table: E x ExpertW4 (device);
 //   active[E], n_active[1], offsets[E+1] from hn_moe_permute; h_ws [rows, I];
 //   y_perm [rows, H]; work = hn_skinny_workspace_bytes(3, rows, H, I, E) bytes.
@@ -1016,11 +1022,11 @@ extern "C" int hn_moe_experts_decode_split_check(long E, long max_rows_per_exper
   return experts_split_ok(E, max_rows_per_expert, rows, H, I, group) ? 0 : 1;
 }
 
-// The experts half of a decode MoE layer: grouped SwiGLU over the routed rows
-// and the ordered, weighted sum back per token.  Where the streaming kernels
-// apply, the down projection runs in four K slices whose fp32 partials (in
-// the workspace) the unpermute sums in slice order (out NULL: left there for
-// the caller); otherwise this is hn_grouped_expert_mlp_int4 into y_ws
+// The experts half of a MoE layer: grouped SwiGLU over the routed rows and the
+// ordered, weighted sum back per token.  Where the streaming kernels apply, or the
+// middle-size kernels with an intermediate size past 4096, the down projection runs
+// in four K slices whose fp32 partials (in the workspace) the unpermute sums in
+// slice order (out NULL: left there for the caller); otherwise this is hn_grouped_expert_mlp_int4 into y_ws
 // followed by hn_moe_unpermute.
 extern "C" int hn_moe_experts_decode(const void* x_perm, const void* table, const int* active,
                                      const int* n_active, const int* offsets, long E,
@@ -1043,7 +1049,7 @@ extern "C" int hn_moe_experts_decode(const void* x_perm, const void* table, cons
                      aligned16(x_perm) && aligned16(h_ws) &&
                      (!mid || !out || (work && work_bytes >= mid_down_bytes(rows, H)));
   HN_ARG_CHECK(out || (split && !shared),
-               "%s: out NULL (partials left for the caller) needs the streaming path with the "
+               "%s: out NULL (partials left for the caller) needs the "
                "K-split down projection (hn_moe_experts_decode_split_check) and no shared "
                "expert", who);
   if (split) {

@@ -22,8 +22,8 @@
 //    four v_mfma_f32_16x16x32_f16.  Two register buffers: stage s + 1
 //    is in flight while stage s (128 k) computes.
 //  * Activations go L2 -> LDS directly (buffer_load ... lds) into two stage
-//    slots, rows XOR-swizzled by 16-byte chunk so the A reads are free of bank
-//    conflicts; one barrier per stage.
+//    slots, rows XOR-swizzled by 16-byte chunk (1.4 to 2.5 bank conflict cycles per
+//    LDS instruction are left); one barrier per stage.
 //  * Where the tiles alone would leave CUs idle, K is split over the waves of a
 //    workgroup (mid_kwave_kernel), or over workgroups where that does not apply: the
 //    splits store fp32 partials, and the last of a tile to arrive (per wave,
@@ -157,7 +157,7 @@ struct Item {
 
 // What a tile's loads need.
 struct TileSrc {
-  const void* px; int nx;     // activation rows of the tile from this split's first k, bytes
+  const void* px; int nx;     // activation rows of the tile, from k = 0; their bytes
   const void* pq[2]; int nq;  // packed matrices
   uint32_t vq[kTN];           // lane byte offsets (out-of-range rows: kOOB)
 };
@@ -645,17 +645,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // One problem of few tiles: K split over the eight waves of a workgroup.
 //
 // A K split over workgroups costs about 8 us of its own (partials out to memory,
-// counter, read back: 64 x 6144 x 4096 takes 22.8 us in 4 splits of 8 stages and
-// 31.1 us in one of 32), and a workgroup of a short K has little in flight.  So a
-// workgroup takes a tile of 64 weight rows x 32 tokens whole and its waves a K
+// counter, read back: 17 x 4096 x 512 in two splits 15.5 us, whole 7.6), and a
+// workgroup of a short K has little in flight.  So a workgroup takes a tile of 64 weight rows x 32 tokens whole and its waves a K
 // range each: every wave stages its own activations (no barrier in the K loop, two
 // slots as above) and the partials meet in LDS, summed in K order.  The
 // activations are read once per 64 weight rows instead of once per 256, from L2.
-// us before / now: 64 x 6144 x 4096 24.9 / 11.8, 64 x 4096 x 1408 19.0 / 6.9,
-// 37 x 4096 x 14336 34.1 / 29.2, 333 x 4096 x 4096 group 64 44.4 / 28.9.  Bound by
-// the stages' latency (about 1.7 us each at 14 per wave); a third register buffer of
-// weights, two stages ahead, gave nothing (32.9 against 32.7 at 128 x 4096 x 14336,
-// 12.6 against 11.9 at 64 x 6144 x 4096).
+// us with K over workgroups (32-token tiles) / over waves: 64 x 6144 x 4096 19.5 /
+// 11.3, 64 x 4096 x 1408 15.0 / 6.8, 333 x 4096 x 4096 group 64 (whole) 36.9 / 30.3, 37
+// x 4096 x 14336 27.8 / 30.0.  Bound by the stages' latency: 27 us for the 14 of a wave
+// at 37 x 4096 x 14336, in which waves issue vector instructions for 28 % of their
+// cycles, wait for 63 %, and the matrix cores are busy for 6 %; a third register
+// buffer of weights, two stages ahead, gave nothing (32.9 against 32.7 at 128 x 4096 x
+// 14336, 12.6 against 11.9 at 64 x 6144 x 4096).
 // ---------------------------------------------------------------------------
 constexpr int kKWaves = 8;
 constexpr int kKScales = 16;                       // scales per row of a wave's K range at most
@@ -855,14 +856,15 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // Resident workgroups of mid_kernel: two per CU.
 int slots() { return 2 * hn_device_cus(); }
 
-// Single problems.  Work in units of one tile's stage.  Measured on MI355X
-// (graph replays over rotating weights, us, 32- / 64-token tiles at their best
-// split against the 256-token GEMM, or the split-K kernels at 64 tokens):
-//   M    64  N  6144 K  4096    20 /  30   39      M 64  N 4096 K 14336   27 /  37  103
-//   M   128  N  4096 K 14336    38 /  45   66      M 333 N 4096 K 14336  100 /  81  129
-//   M  1024  N  4096 K 14336   206 / 161  158      M 200 N 14336 x2       98 /  81  102
-//   M   333  N 14336 K 4096 x2 146 / 140  138      M 1024 N 4096 K 1408   26 /  40   49
-//   M   512  N  4096 K 4096 g64 41 /  37   75      M 1024 N 1408 K 4096   35 /  50   76
+// Single problems that mid_kernel takes.  Work in units of one tile's stage.  Measured
+// on MI355X (graph replays over rotating weights, us, 32- / 64-token tiles, the
+// 256-token GEMM or, at 64 tokens, the split-K kernels; M x N x K):
+//     64 x  6144 x  4096     20 /  28    39      64 x 4096 x 14336       29 /  43   102
+//    128 x  4096 x 14336     39 /  43    64     333 x 4096 x 14336       90 /  84   128
+//   1024 x  4096 x 14336    174 / 151   152     200 x 14336 x 4096 x2    98 /  77    98
+//    333 x 14336 x 4096 x2  146 / 146   139    1024 x 4096 x 1408        25 /  29    48
+//    512 x  4096 x 4096 g64  38 /  44    75    1024 x 1408 x 4096        32 /  43    75
+//    300 x 14336 x 4096      92 /  71   106     600 x 4096 x 4096        48 /  48    81
 // so: 32-token tiles up to 8192 units (16 stages per resident workgroup), then
 // 64-token tiles while they fit one round of workgroups and 16384 units, past
 // which the weights' re-reads and unpacks cost more than the GEMM's tile
@@ -1024,6 +1026,7 @@ void launch_single(const MidArgs& A, const MidPlan& p, int grid, hipStream_t s) 
 // average, 58 at most, 166 + 107 against 150 + 89; 128 experts of 4096 x 1408 with 19
 // rows 196 + 120 against 205 + 129).
 constexpr long kRows32 = 20;
+constexpr long kGroupedStages = 32;  // of an item at most: the sizes that were measured
 
 }  // namespace
 
@@ -1116,7 +1119,7 @@ extern "C" int hn_mid_grouped_impl(int phase, const void* x, long ld_x, const vo
                                    long ld_o, float* part, int ks, void* stream, int dry_run) {
   const long K = phase == 0 ? H : I, N = phase == 0 ? I : H;
   if (E < 1 || E > kMaxProb || group != kStageK || K % kStageK != 0 || ks < 1 ||
-      (K / kStageK) % ks != 0 || K / kStageK / ks > kMaxScales)
+      (K / kStageK) % ks != 0 || K / kStageK / ks > kGroupedStages)
     return HN_NOT_HANDLED;
   if ((phase == 0 && part) || N * (K / 2) >= (long)kOOB || N * (K / group) * 2 >= (long)kOOB ||
       ld_x * 2 * 64 >= (long)kOOB || ld_x % 8 != 0)

@@ -83,15 +83,7 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const h16* __restric
   if (lane == 0) logits[(long)t * E + e] = acc;
 }
 
-// One wave per token (more than 16 experts) or one thread per token.
-// Group-limited selection of GLM4SigmoidRouter (model/glm4.py:285-298), one
-// wave per token: the experts' sigmoids (sigmoid_f32, as the top-k) go to
-// LDS, lane g < n_group takes the max over its group of E / n_group
-// consecutive experts, the topk_group largest group scores are kept (equal
-// scores: the lower group), and the row is written back with -inf for every
-// expert of the other groups (their sigmoid is then exactly 0, the
-// reference's masked score).
-// The same sums for many dot products: a wave takes LT tokens x 4 experts, so
+// router_logits_kernel's sums for many dot products: a wave takes LT tokens x 4 experts, so
 // a row is read once for several products.  Each sum keeps its order (per lane,
 // then pairs 32, 16, .. 1 apart; a pair's two sums are the same number), so the
 // bits are router_logits_kernel's: the first steps halve the sums each lane
@@ -152,6 +144,13 @@ __global__ __launch_bounds__(256) void router_logits_tile_kernel(
 }
 constexpr long kLogTileMin = 16384;  // products
 
+// Group-limited selection of GLM4SigmoidRouter (model/glm4.py:285-298), one
+// wave per token: the experts' sigmoids (sigmoid_f32, as the top-k) go to
+// LDS, lane g < n_group takes the max over its group of E / n_group
+// consecutive experts, the topk_group largest group scores are kept (equal
+// scores: the lower group), and the row is written back with -inf for every
+// expert of the other groups (their sigmoid is then exactly 0, the
+// reference's masked score).
 __global__ __launch_bounds__(256) void router_group_limit_kernel(
     const float* __restrict__ logits, int T, int E, int n_group, int topk_group,
     float* __restrict__ out) {
@@ -184,6 +183,7 @@ __global__ __launch_bounds__(256) void router_group_limit_kernel(
     out[(long)t * E + e] = s_keep[wv][e / gsz] ? l[e] : -__builtin_inff();
 }
 
+// One wave per token (more than 16 experts) or one thread per token.
 __global__ __launch_bounds__(256) void router_topk_kernel(
     const float* __restrict__ logits, const float* __restrict__ bias, int T, int E, int k,
     int mode, float eps, float scaling, int* __restrict__ idx_out, h16* __restrict__ w_out) {

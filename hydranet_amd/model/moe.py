@@ -225,8 +225,8 @@ def decode_layer_fits(T: int, E: int, k: int, table: "ExpertTable", gate_w: torc
 
 
 def experts_split_fits(T: int, k: int, table: "ExpertTable") -> bool:
-    """Whether moe_dispatch at decode takes the streaming path with the K-split
-    down projection (then it can fold the next RMSNorm into its unpermute)."""
+    """Whether moe_dispatch at decode runs the down projection in K slices
+    (then it can fold the next RMSNorm into its unpermute)."""
     H, I, g = table.dims
     return T <= _lib.DECODE_MAX_ROWS and _lib.lib().hn_moe_experts_decode_split_check(
         table.num_experts, T, T * k, H, I, g) == 0
@@ -359,8 +359,8 @@ def moe_experts_forward(hidden: torch.Tensor, idx: torch.Tensor, w: torch.Tensor
               _lib.ptr(x_perm), H, n, H, st)
     h_ws = torch.empty((max(n, 1), I), dtype=torch.float16, device=dev)
     y_perm = torch.empty((max(n, 1), H), dtype=torch.float16, device=dev)
-    # above DECODE_MAX_ROWS tokens the grouped prefill GEMM runs, its workspace
-    # holding the stream-K counters and partial sums
+    # above DECODE_MAX_ROWS tokens: the middle-size kernels or, by the rows per expert,
+    # the prefill GEMM, whose workspace holds the split sums of either
     work = (_lib.skinny_workspace(3, n, H, I, E, dev) if T <= _lib.DECODE_MAX_ROWS
             else _lib.gemm_workspace(dev))
     _lib.call("hn_grouped_expert_mlp_int4", _lib.ptr(x_perm), _lib.ptr(table.dev),

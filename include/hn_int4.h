@@ -39,22 +39,27 @@ int hn_int4_dequant(const void* packed, long ld_p, const void* scales, long ld_s
 int hn_int4_quantize(const void* w, long ld_w, int dtype, int mode, void* packed, long ld_p,
                      void* scales, long ld_s, long N, long K, long group, void* stream);
 
-/* Workspace bytes for the skinny (decode) kernels below.  kind 0: hn_int4_linear
- * (M, N, K); 1: hn_int4_gate_up_silu (M, N=I, K=H); 2: hn_expert_mlp_int4
- * (M=T, N=H, K=I); 3: hn_grouped_expert_mlp_int4 (M=rows, N=H, K=I, E).  The
- * workspace must be zero-filled once when allocated; the kernels leave its
+/* Workspace bytes of the entry points below at decode sizes, up to 64 rows per
+ * weight matrix (above, hn_gemm_workspace_bytes; M past 64 counts as 64 but for
+ * kind 3): K splits of the decode and middle-size kernels.  kind 0:
+ * hn_int4_linear (M, N, K); 1: hn_int4_gate_up_silu (M, N=I, K=H); 2:
+ * hn_expert_mlp_int4 (M=T, N=H, K=I); 3: hn_grouped_expert_mlp_int4 (M=rows, N=H,
+ * K=I, E).  The workspace must be zero-filled once when allocated; the kernels leave its
  * counters at zero.  Its layout (counters in the first 2 MiB, partials after)
  * is the same for every call, so one buffer may serve calls of every kind and
  * size in turn.  Calls that run concurrently need distinct workspaces.
  * No counterpart in the reference (Triton needs no split-K workspace). */
 long hn_skinny_workspace_bytes(int kind, long M, long N, long K, long E);
 
-/* Workspace bytes of the prefill (MFMA GEMM) kernels' stream-K split: fp32
- * partial slots for two tile segments per workgroup plus per-(tile, wave)
- * counters.  Passed (zero-filled once; the kernels leave the counters at zero)
- * as the work argument of the entry points below at prefill sizes, it lets
+/* Workspace bytes of the entry points below above 64 rows per weight matrix: the
+ * prefill (MFMA GEMM) kernels' stream-K split (fp32 partial slots for two tile
+ * segments per workgroup plus per-(tile, wave) counters), and the middle-size
+ * kernels' K splits, which are only made where they fit it: a larger buffer changes
+ * nothing.  Optional there: with less, or NULL, products whose K would be split run
+ * by the GEMM in whole tiles.  Passed (zero-filled once; the kernels leave the
+ * counters at zero) as the work argument, it lets the GEMM have
  * the tiles short of a whole round over the CUs (and the experts' last,
- * shorter M-tiles) be split over every CU by cost-weighted (tile, k-chunk)
+ * shorter M-tiles) split over every CU by cost-weighted (tile, k-chunk)
  * iterations, tiles split at the shares' ends being summed in a fixed order
  * by the last segment to finish.  No counterpart in the reference (Triton's
  * GEMM takes no workspace). */
@@ -63,7 +68,11 @@ long hn_gemm_workspace_bytes(void);
 /* out[M, N] = fp16(x[M, K] @ deq(W)^T), fp32 accumulation.  Replaces the
  * int4_matmul_kernel launch in int4_gemm.int4_linear (kernels/int4_gemm.py:124-172)
  * and int4_expert_mlp.int4_linear (kernels/int4_expert_mlp.py:99-156).
- * K % 32 == 0, group a multiple of 32 dividing K, 16-byte aligned rows. */
+ * K % 32 == 0, group a multiple of 32 dividing K, 16-byte aligned rows of x
+ * and wq.  By M: the streaming and split-K kernels up to
+ * 16 rows; the middle-size kernels from 17 to a few hundred (K a multiple of 128,
+ * group 32, 64 or 128); the split-K kernels up to 64 and the prefill GEMM above where
+ * those do not take a product or are slower. */
 int hn_int4_linear(const void* x, long ld_x, const void* wq, long ld_q, const void* ws, long ld_s,
                    void* out, long ld_o, long M, long N, long K, long group, void* work,
                    long work_bytes, void* stream);
@@ -156,17 +165,21 @@ int hn_moe_unpermute(const void* y_perm, long ld_y, const int* inv, const int* i
                      long T, long k, const void* shared, long ld_sh, void* out, long ld_o, long H,
                      void* stream);
 
-/* Grouped SwiGLU over every active expert of one MoE layer in two launches:
- * the decode kernels up to 64 rows per expert, the MFMA GEMM kernels above
- * (which take no workspace: it may then be NULL / 0 bytes).  x_perm [rows, H] sorted by expert; table: E x
+/* Grouped SwiGLU over every active expert of one MoE layer.  max_rows_per_expert
+ * bounds any expert's rows (e.g. the layer's tokens); by it and by the rows per
+ * expert on average the streaming kernels run (up to 16 rows; up to 64 with 10 on
+ * average), the middle-size kernels (up to 128 on average; group 128, H a multiple of
+ * 128 up to 4096, I up to 4096 or a multiple of 512 up to 16384), the split-K kernels
+ * (other shapes up to 64 rows) or the prefill GEMM: two launches, three where the
+ * middle-size kernels run the down projection in K slices (I past 4096).  x_perm [rows, H] sorted by expert; table: E x
  * {gate_q, gate_s, up_q, up_s, down_q, down_s} device pointers (u64), each
  * 16-byte aligned (GpuExpertSlot slabs are); active /
  * n_active / offsets from hn_moe_permute; h_ws [rows, I] fp16 buffer;
  * y_perm [rows, H] fp16 out; work: hn_skinny_workspace_bytes(3, rows, H, I, E),
- * zero-filled once.  Above 64 rows per expert (the MFMA GEMM kernels) work
- * may instead hold hn_gemm_workspace_bytes() bytes, which enables their
- * stream-K split of the remainder tiles over the CUs, or be NULL (whole
- * tiles go round-robin).
+ * zero-filled once.  With max_rows_per_expert above 64, work may instead hold
+ * hn_gemm_workspace_bytes() bytes, which enables the GEMM's stream-K split of the
+ * remainder tiles over the CUs and the middle-size kernels' K slices, or be NULL
+ * (the GEMM's whole tiles go round-robin, also for layers that would be sliced).
  * Replaces the per-expert loop calling expert_mlp_int4_fused
  * (model/mixtral.py:327-354, model/glm4.py:421-455). */
 int hn_grouped_expert_mlp_int4(const void* x_perm, const void* table, const int* active,
@@ -177,12 +190,12 @@ int hn_grouped_expert_mlp_int4(const void* x_perm, const void* table, const int*
 
 /* The experts half of a MoE layer at decode: hn_grouped_expert_mlp_int4 plus
  * hn_moe_unpermute (same arguments; inv / idx / w / shared as for
- * hn_moe_unpermute, out [T, H]).  Where the streaming kernels apply, the down
- * projection runs in four K slices whose fp32 partials (kept in work) the
- * unpermute adds in slice order before the fp16 rounding; y_ws [rows, H] fp16
- * is then unused.  work: hn_skinny_workspace_bytes(3, rows, H, I, E).  out
- * NULL (only on that streaming path, hn_moe_experts_decode_split_check, and
- * without a shared expert): no unpermute; the partials stay in work at byte
+ * hn_moe_unpermute, out [T, H]).  Where the streaming kernels apply, or the
+ * middle-size kernels with I past 4096, the down projection runs in four K slices
+ * whose fp32 partials (kept in work) the unpermute adds in slice order before the
+ * fp16 rounding; y_ws [rows, H] fp16 is then unused.  work: as for
+ * hn_grouped_expert_mlp_int4.  out NULL (only with the down projection in slices,
+ * hn_moe_experts_decode_split_check, and without a shared expert): no unpermute; the partials stay in work at byte
  * hn_moe_decode_layer_partials(T, E, k, H, I) for the caller (e.g.
  * hn_unpermute_add_rmsnorm).
  * Replaces the per-expert loop and index_add_ of MixtralMoELayer.forward
@@ -194,8 +207,7 @@ int hn_moe_experts_decode(const void* x_perm, const void* table, const int* acti
                           long T, long k, const void* shared, long ld_sh, void* out, long ld_o,
                           void* work, long work_bytes, void* stream);
 
-/* 0 when hn_moe_experts_decode takes its streaming path with the K-split down
- * projection for (E, max_rows_per_expert, rows, H, I, group) under the current
+/* 0 when hn_moe_experts_decode runs the down projection in K slices for (E, max_rows_per_expert, rows, H, I, group) under the current
  * decode kernel family (then out may be NULL), else a nonzero code (no
  * message set). */
 int hn_moe_experts_decode_split_check(long E, long max_rows_per_expert, long rows, long H,
@@ -430,10 +442,11 @@ int hn_rope_append(const void* q, long ld_q, const void* k, long ld_k, const voi
 /* Decode kernel family for hn_int4_linear, hn_int4_gate_up_silu,
  * hn_expert_mlp_int4 and hn_grouped_expert_mlp_int4, for the calling thread
  * only (each thread starts at 0; a switch never affects another thread):
- *   0  automatic: the persistent streaming kernels for group 128 and at most
- *      16 rows per weight matrix, the split-K kernels otherwise (default);
- *   1  split-K kernels only.
- * Both give the same results to within fp32 summation order.  No counterpart
+ *   0  automatic (default): the kernels named at each entry point;
+ *   1  the split-K kernels up to 64 rows per weight matrix, the prefill GEMM above.
+ * Both give the same results to within fp32 summation order, but that the prefill
+ * GEMM, and every kernel below group 128, rounds each scaled weight to fp16 (2^-11)
+ * where the others scale fp32 sums.  No counterpart
  * in the reference; for A/B measurement and tests. */
 int hn_set_decode_path(int path);
 

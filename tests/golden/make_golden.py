@@ -1,6 +1,6 @@
 """Write the golden vectors in tests/golden/ by running the REFERENCE's own code.
 
-Run in the build container only (the reference tree is not on the GPU box):
+Run where the reference tree is mounted:
 
     python tests/golden/make_golden.py /root/reference
     python tests/golden/make_golden.py /root/reference grouped_router   # one fixture
