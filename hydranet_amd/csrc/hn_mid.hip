@@ -32,7 +32,7 @@
 //  * Group scales: SC multiplies the fp32 partial of each 128-k group (group a
 //    multiple of 128); otherwise each unpacked weight is multiplied in fp16 and
 //    rounded once, the reference's dequantised weight.
-#include "hn_common.h"
+#include "hn_lds_dma.h"
 
 namespace {
 
@@ -71,50 +71,6 @@ struct MidArgs {
   unsigned long long* ctr;  // SUM: [tiles][kWaves] tagged counters, left zero
   unsigned long long tag;
   uint32_t m_pair, magic;
-};
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, bytes, 0x00020000);
-}
-
-__device__ __forceinline__ lds_void_t* lds_ptr(uint32_t addr) {
-  return (lds_void_t*)((__attribute__((address_space(3))) char*)nullptr + addr);
-}
-
-__device__ __forceinline__ void dma_b128(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff,
-                                         uint32_t lds) {
-  // soffset and the LDS address are uniform by construction
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds_ptr(__builtin_amdgcn_readfirstlane(lds)), 16,
-                                           voff, __builtin_amdgcn_readfirstlane(soff), 0, 0);
-}
-
-template <typename T>
-__device__ __forceinline__ T lds_read(uint32_t addr) {
-  return *reinterpret_cast<const __attribute__((address_space(3))) T*>(
-      (__attribute__((address_space(3))) char*)nullptr + addr);
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
-}
-
-// Barrier of the K loop (as hn_gemm.hip's): LDS reads returned, the loads of
-// later stages still in flight.
-__device__ __forceinline__ void stage_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-struct DeqRegs {
-  uint32_t m_pair;  // SGPR 0x00F0000F: low nibble of byte 0, high nibble of byte 2
-  uint32_t magic;   // 0x64006400
-  uint32_t mul;     // half2(1, 1/16)
-  uint32_t add;     // half2(-1032, -72)
 };
 
 // Eight exact fp16 (n_k - 8), k = 0..7 in order, from one packed dword; with
